@@ -230,18 +230,24 @@ int mrsa_route_topk_fwd(const void* q, const void* lmk, const float* lse_local,
  * The same reference call sites; the decode caller is route_topk_g7 at
  * dream_dllm_hils/fastdllm_attention.py:299-314 (32 query rows against the
  * whole cache).
- *   - Shapes of the matrix-core kernel (head_dim 128, groups 7 or 8,
- *     chunks <= 256, topk <= 64, bf16 scores, not causal): a workspace of
- *     at least batch * seq_len * kv_heads * groups * chunks * 2 bytes holds
- *     the bf16 raw scores of every chunk, so the kernel runs one pass and
- *     gathers the picks' scores from it instead of recomputing them.
+ *   - Shapes of the one-pass kernel (head_dim 128, groups <= 8, chunks <= 256,
+ *     topk <= 64, bf16 scores, not causal) take no workspace.
+ *   - 4096 or more rows (batch * seq_len * kv_heads) with head_dim 128,
+ *     groups <= 8, chunks <= 4096 and topk <= 64: the selection scores
+ *     [batch, seq_len, kv_heads, chunks rounded up to 16] go through the fp32
+ *     workspace, with each head's LSE total.
  *   - Otherwise, with mrsa_route_topk_workspace_bytes() bytes and
  *     head_dim == 128, groups <= 8, chunks <= 4096, the logits of all rows are
  *     computed on the matrix cores into the fp32 workspace and selected by a
  *     second kernel, one workgroup per (row, KV head).
  * Other shapes (and a smaller workspace) take mrsa_route_topk_fwd's paths.
  * Same results either way.
+ * mrsa_route_topk_needed_bytes: the bytes of the path the call takes (0: it
+ * takes none).
  */
+int64_t mrsa_route_topk_needed_bytes(int64_t batch, int64_t seq_len, int64_t chunks,
+                                     int64_t kv_heads, int64_t groups, int64_t head_dim,
+                                     int64_t topk, int is_causal, int scores_fp32);
 int64_t mrsa_route_topk_workspace_bytes(int64_t batch, int64_t seq_len, int64_t chunks,
                                         int64_t kv_heads, int64_t groups);
 int mrsa_route_topk_ws_fwd(const void* q, const void* lmk, const float* lse_local,

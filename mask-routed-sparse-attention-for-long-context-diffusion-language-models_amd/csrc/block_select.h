@@ -158,19 +158,33 @@ struct BlockSelect {
   }
 };
 
+// Wave reductions of integers on DPP lane moves and row swaps (no LDS round
+// trip: a search starts with three of them).  Every lane must be active.
+__device__ __forceinline__ uint32_t wave_min_u(uint32_t v) {
+  v = group8_min_u(v);
+  v = min(v, (uint32_t)dpp_mov_i<0x140>((int)v));  // row_mirror
+  const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+  const uint32_t s = min((uint32_t)r[0], (uint32_t)r[1]);
+  const auto q = __builtin_amdgcn_permlane16_swap(s, s, false, false);
+  return min((uint32_t)q[0], (uint32_t)q[1]);
+}
+__device__ __forceinline__ uint32_t wave_max_u(uint32_t v) {
+  return ~wave_min_u(~v);
+}
+__device__ __forceinline__ int wave_sum_dpp(int v) {
+  v = group8_sum_i(v);
+  v += dpp_mov_i<0x140>(v);
+  const auto r = __builtin_amdgcn_permlane32_swap((uint32_t)v, (uint32_t)v, false, false);
+  const int s = (int)r[0] + (int)r[1];
+  const auto q = __builtin_amdgcn_permlane16_swap((uint32_t)s, (uint32_t)s, false, false);
+  return (int)q[0] + (int)q[1];
+}
+
 // The same selection by one wave with no barrier: element (i, lane) has
 // order index i * 64 + lane; every count is a sum of ballot popcounts, so
 // the whole search runs on scalar registers after each compare.
 template <int PER>
 struct WaveSelect {
-  __device__ static uint32_t wave_min_u(uint32_t v) {
-    for (int o = 1; o < 64; o <<= 1) v = min(v, (uint32_t)__shfl_xor((int)v, o, 64));
-    return v;
-  }
-  __device__ static uint32_t wave_max_u(uint32_t v) {
-    for (int o = 1; o < 64; o <<= 1) v = max(v, (uint32_t)__shfl_xor((int)v, o, 64));
-    return v;
-  }
   // Ballots in groups of 8 with a scheduling fence between groups: the
   // scheduler would otherwise keep all PER ballot masks live in SGPRs.
   __device__ static int count_ge(const uint32_t (&key)[PER], int n, uint32_t t) {
@@ -203,7 +217,7 @@ struct WaveSelect {
         kmax = max(kmax, key[i]);
       }
     }
-    for (int o = 1; o < 64; o <<= 1) nfin += __shfl_xor(nfin, o, 64);
+    nfin = wave_sum_dpp(nfin);
     kmin = wave_min_u(kmin);
     kmax = wave_max_u(kmax);
     thr_tie = 0u;

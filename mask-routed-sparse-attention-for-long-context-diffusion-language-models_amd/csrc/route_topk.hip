@@ -12,13 +12,16 @@
 // selection score go to the lower chunk index (the rule of the reference's
 // fused selection kernel, topk_head_softmax.py:614-626).
 //
-// Fast path (route_topk_fast_kernel): head_dim 128, chunks <= 256, bf16
-// scores, 7 or 8 heads per KV group, no workspace.  A workgroup holds 128
-// queries of one KV head (16 per wave); pass 1 computes every head's logits
-// on the matrix cores and folds them into the running max over heads, the
-// K-th largest score of each query is found by bisection on order-preserving
-// integer keys (exact ties at the threshold broken by chunk index), and
-// pass 2 recomputes the logits for the picks' raw scores.
+// One-pass path (route_heads_kernel, route_tile_kernel): head_dim 128, chunks
+// <= 256, bf16 scores, up to 8 heads per KV group, no workspace.  Either a
+// workgroup holds 16 or 32 queries of one KV head with one or two waves per
+// head, whose logits stay in registers while the maxima over heads are
+// selected from, or each of its waves takes 16 queries through every head in
+// two passes.
+//
+// Scan path (route_lse_kernel, route_scan_kernel and route_pick_kernel, with a
+// caller workspace): many rows against up to 4096 chunks; the selection scores
+// pass through the workspace and the picks' raw scores are formed again.
 //
 // Short-block path (route_logits_kernel + route_select_kernel, with a caller
 // workspace): logits of few query rows against up to 4096 chunks on the
@@ -58,7 +61,8 @@ struct RouteArgs {
   int32_t* indices;
   void* scores;
   int scores_fp32;
-  int vec_out;  // K % 32 == 0, indices and scores 16-byte aligned: one 16-byte store per lane
+  int vec32_out;  // K % 32 == 0, indices and scores 16-byte aligned: 16-byte stores of both
+  int vec_out;  // K % 8 == 0 and the scores 16-byte aligned: stores of 8 or 16 bytes
 };
 
 __device__ __forceinline__ int64_t floor_div(int64_t a, int64_t b) {
@@ -102,7 +106,358 @@ __device__ __forceinline__ const uint16_t* lmk_row(const RouteArgs& a, int64_t b
 }
 
 // ---------------------------------------------------------------------------
-// Fast path.
+// One-pass path (C <= 256): a wave per head.
+//
+// A workgroup of 8 waves holds 16 QT queries of one KV head; wave g computes
+// head g's logits S^T = lmk . q^T, NT 16-chunk tiles (16 chunks x 16 queries
+// per matrix product: lane (j, grp) holds query j's chunks 16 t + 4 grp + i),
+// and keeps them in registers, so each logit is formed once:
+//   scores  the head's LSE over all chunks (the four lanes sharing j), then
+//           x - logaddexp(local LSE, LSE) into the workgroup's [chunk][query]
+//           maxima with LDS float-max atomics;
+//   picks   each wave selects 2 QT queries' K largest, lanes over chunks, and
+//           lists them in LDS;
+//   output  the scoring waves write their bf16 raw logits to LDS (over the
+//           maxima, dead by then) and gather them at the picks.
+// A wave's landmark rows stream through its own ring of 16-chunk LDS slots,
+// filled by DMA and read with no workgroup barrier.
+//
+// Bound: a chain of short phases (loads, products, three passes over the
+// logits, selection, output) rather than any one unit, so what counts is how
+// many waves share a phase and how many workgroups share a CU.  Each workgroup
+// reads all G C landmark rows from L2 (458 KB at G = 7, C = 256): 32 queries
+// (QT = 2) halve that, 16 (QT = 1) give a short sequence twice the workgroups.
+// ---------------------------------------------------------------------------
+constexpr int kHeadThreads = 512;
+constexpr int kHeadWaves = kHeadThreads / 64;
+constexpr int kHeadRing = 2;   // landmark tiles in flight per wave
+constexpr int kFastMaxTopk = 64;
+constexpr int kFastMaxChunks = 256;
+
+typedef __attribute__((address_space(3))) void lds_void_t;
+
+// logaddexp(local LSE, LSE of the logits) from the latter in base 2.  A -inf
+// total (no visible logit at all) is clamped to -FLT_MAX: finite x - tot then
+// ties at the top like x - (-inf) = +inf would, and -inf stays.
+__device__ __forceinline__ float route_total(float lse, float lse2) {
+  const float lv2 = lse * kLog2e;
+  const float hi = fmaxf(lv2, lse2), lo = fminf(lv2, lse2);
+  return hi == neg_inf() ? -__FLT_MAX__ : (hi + log2_hw(1.f + exp2_hw(lo - hi))) * kLn2;
+}
+
+__device__ __forceinline__ void lds_max(float* p, float v) {
+  __hip_atomic_fetch_max(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+// Buffer resource of one batch's landmark keys (under 2 GB on the paths that
+// use it), read by 24-bit lane offsets with the head slot in the scalar offset.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t lmk_rsrc(const RouteArgs& a, int64_t b,
+                                                           uint32_t rowlen) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(a.lmk + b * a.C * (int64_t)rowlen),
+                                           (short)0, (int)((uint32_t)a.C * rowlen * 2u),
+                                           0x00020000);
+}
+
+template <int NT, int QT>
+struct HeadsLayout {
+  static constexpr int kQ = 16 * QT;           // queries
+  static constexpr int kC = 16 * NT;           // chunks, padded
+  static constexpr int kPitch = kQ + 4;        // floats per chunk of the maxima (4 mod 16: the
+                                               // four lane groups meet distinct banks)
+  static constexpr int kStage = kHeadRing * 4096;  // ring bytes per wave
+  static constexpr int kRaw = kQ * kC * 2;         // raw-logit bytes per head
+  static constexpr int kMax = kC * kPitch * 4;
+  // One region holds the rings, then the maxima, then the raw logits; after
+  // it the bias rows [G][kC], the pick lists [kQ][K] int16 and the chunk flags
+  // [kC].
+  static int bias(int G) {
+    int n = G * kStage;
+    if (n < G * kRaw) n = G * kRaw;
+    return n < kMax ? kMax : n;
+  }
+  static int picks(int G) { return bias(G) + G * kC * 4; }
+  static size_t total(int G, int K) { return (size_t)picks(G) + kQ * K * 2 + kC; }
+};
+
+template <int NT, int QT>
+__global__ void __launch_bounds__(kHeadThreads, 4)
+    route_heads_kernel(RouteArgs a, int bias_at, int picks_at) {
+  using Lay = HeadsLayout<NT, QT>;
+  constexpr int kQ = Lay::kQ, kC = Lay::kC, kPitch = Lay::kPitch;
+  constexpr int kPer = NT / 4;        // chunks per selecting lane
+  constexpr int kRows = kQ / kHeadWaves;  // queries a wave selects for
+  static_assert(kPer * 64 == kC && kRows >= 1, "whole lanes and rows");
+  extern __shared__ __align__(16) unsigned char smem[];
+  const int G = a.G, K = a.K;
+  float* mx_s = reinterpret_cast<float*>(smem);
+  int16_t* picks = reinterpret_cast<int16_t*>(smem + picks_at);
+  unsigned char* cbad = smem + picks_at + kQ * K * 2;
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int j = lane & 15, grp = lane >> 4;
+  const int64_t b = blockIdx.z;
+  const int h = blockIdx.y;
+  const int64_t L = a.L;
+  const int C = (int)a.C;
+  const int64_t q0 = (int64_t)blockIdx.x * kQ;
+  const int g = wave;          // head of this wave's scores
+  const bool scoring = g < G;  // wave-uniform
+
+  // Every load of the prologue in flight together: the queries, their local
+  // LSE and the head's bias; the flags of the chunk this thread looks at (the
+  // last slot of a chunk is its landmark); an explicit drop mask's entries for
+  // the rows and chunks this lane selects from.
+  u32x4_t Q[QT][4];
+  float lse[QT], bv[kPer];
+  const int gl = min(g, G - 1);
+#pragma unroll
+  for (int u = 0; u < QT; ++u) {
+    // rows past L re-read row L - 1
+    const int64_t qrow = ((b * L + min(q0 + 16 * u + j, L - 1)) * a.Hkv + h) * G + gl;
+    const uint16_t* src = a.q + qrow * 128 + 8 * grp;
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) Q[u][ks] = *reinterpret_cast<const u32x4_t*>(src + 32 * ks);
+    lse[u] = a.pre_softmax ? 0.f : a.lse[qrow];
+  }
+#pragma unroll
+  for (int i = 0; i < kPer; ++i)
+    bv[i] = a.bias ? a.bias[((b * C + min(lane + 64 * i, C - 1)) * a.Hkv + h) * G + gl] : 0.f;
+  uint32_t dropbits = 0u;
+  if (a.derive_window >= 0) {
+    if (tid < kC) {
+      bool any = tid < C && a.block_size > 1;
+      if (any && a.key_valid)
+        any = chunk_has_valid_key(a.key_valid + b * L + (int64_t)tid * a.block_size, a.block_size);
+      cbad[tid] = !any;
+    }
+  } else if (a.drop) {
+    int32_t d[kRows][kPer];
+#pragma unroll
+    for (int it = 0; it < kRows; ++it) {
+      const int32_t* drow = a.drop + (b * L + min(q0 + wave * kRows + it, L - 1)) * C;
+#pragma unroll
+      for (int i = 0; i < kPer; ++i) d[it][i] = drow[min(lane + 64 * i, C - 1)];
+    }
+#pragma unroll
+    for (int it = 0; it < kRows; ++it)
+#pragma unroll
+      for (int i = 0; i < kPer; ++i) dropbits |= (uint32_t)(d[it][i] != 0) << (kPer * it + i);
+  }
+
+  // ---- scores ---------------------------------------------------------------
+  f32x4_t S[NT][QT];
+  float* bias_s = reinterpret_cast<float*>(smem + bias_at) + g * kC;
+  float tot[QT];
+  // x = s * scale + bias (-inf past C), formed anew in each of the three
+  // passes over the held logits.
+  auto x_of = [&](int t, int u, const f32x4_t& bt, int i) {
+    return __builtin_fmaf(S[t][u][i], a.sm_scale, bt[i]);
+  };
+  auto bias_of = [&](int t) {
+    return *reinterpret_cast<const f32x4_t*>(bias_s + 16 * t + 4 * grp);
+  };
+  if (scoring) {
+    unsigned char* ring = smem + wave * Lay::kStage;
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) bias_s[lane + 64 * i] = lane + 64 * i < C ? bv[i] : neg_inf();
+    // The loads above complete before the first DMA is in flight: a later wait
+    // for one of them would wait for the ring too.
+#pragma unroll
+    for (int u = 0; u < QT; ++u) {
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks) asm volatile("" : "+v"(Q[u][ks]));
+      asm volatile("" : "+v"(lse[u]));
+    }
+    // Tile t into its slot: 4 instructions of 4 rows x 256 bytes.  Part p of
+    // row r sits at unit p ^ r of the row.  Rows >= C re-read row C - 1 (their
+    // bias is -inf).
+    const uint32_t rowlen = (uint32_t)(a.per_head_lmk ? a.Hkv * G : a.Hkv) * 128u;
+    const uint32_t head = 256u * (uint32_t)(a.per_head_lmk ? h * G + g : h);
+    const __amdgpu_buffer_rsrc_t lrs = lmk_rsrc(a, b, rowlen);
+    auto stage = [&](int t) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const int r = 4 * k + grp;
+        const uint32_t c = (uint32_t)min(16 * t + r, C - 1);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(
+            lrs, (lds_void_t*)(ring + (t % kHeadRing) * 4096 + 1024 * k), 16,
+            2u * (__umul24(c, rowlen) + 8u * (uint32_t)(j ^ r)), head, 0, 0);
+      }
+    };
+#pragma unroll
+    for (int t = 0; t < kHeadRing; ++t) stage(t);
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      static_assert(kHeadRing == 2, "one tile (4 loads) is in flight behind the awaited one");
+      if (t + 1 < NT) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+      else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      const unsigned char* arow = ring + (t % kHeadRing) * 4096 + j * 256;
+      u32x4_t A[4];
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks)
+        A[ks] = *reinterpret_cast<const u32x4_t*>(arow + (((4 * ks + grp) ^ j) * 16));
+#pragma unroll
+      for (int u = 0; u < QT; ++u) {
+        S[t][u] = zero4();
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) S[t][u] = mfma_bf16_16x16x32(A[ks], Q[u][ks], S[t][u]);
+      }
+      if (t + kHeadRing < NT) {
+        // the slot's reads are done before its next tile is requested
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        stage(t + kHeadRing);
+      }
+    }
+    // LSE over all chunks in base 2 with the hardware exp2 / log2.  With every
+    // x -inf the stabiliser is 0 and the sum 0.
+#pragma unroll
+    for (int u = 0; u < QT; ++u) tot[u] = 0.f;
+    if (!a.pre_softmax) {  // uniform
+      float m[QT], m2[QT], part[QT], p[QT][4];
+#pragma unroll
+      for (int u = 0; u < QT; ++u) {
+        m[u] = neg_inf();
+#pragma unroll
+        for (int i = 0; i < 4; ++i) p[u][i] = 0.f;
+      }
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        const f32x4_t bt = bias_of(t);
+#pragma unroll
+        for (int u = 0; u < QT; ++u)
+          m[u] = max3_raw(m[u], max_raw(x_of(t, u, bt, 0), x_of(t, u, bt, 1)),
+                          max_raw(x_of(t, u, bt, 2), x_of(t, u, bt, 3)));
+      }
+#pragma unroll
+      for (int u = 0; u < QT; ++u) {
+        m2[u] = across4_max(m[u]) * kLog2e;
+        if (m2[u] == neg_inf()) m2[u] = 0.f;
+      }
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        const f32x4_t bt = bias_of(t);
+#pragma unroll
+        for (int u = 0; u < QT; ++u)
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            p[u][i] += exp2_hw(__builtin_fmaf(x_of(t, u, bt, i), kLog2e, -m2[u]));
+      }
+#pragma unroll
+      for (int u = 0; u < QT; ++u)
+        part[u] = across4_sum((p[u][0] + p[u][1]) + (p[u][2] + p[u][3]));
+#pragma unroll
+      for (int u = 0; u < QT; ++u) tot[u] = route_total(lse[u], m2[u] + log2_hw(part[u]));
+    }
+  }
+  __syncthreads();  // the rings are done
+  for (int i = tid; i < Lay::kMax / 16; i += kHeadThreads) {
+    const float n = neg_inf();
+    reinterpret_cast<f32x4_t*>(mx_s)[i] = f32x4_t{n, n, n, n};
+  }
+  __syncthreads();
+  if (scoring) {
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      const f32x4_t bt = bias_of(t);
+#pragma unroll
+      for (int u = 0; u < QT; ++u)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          lds_max(mx_s + (16 * t + 4 * grp + i) * kPitch + 16 * u + j,
+                  x_of(t, u, bt, i) - tot[u]);
+    }
+  }
+  __syncthreads();
+
+  // ---- picks ----------------------------------------------------------------
+  const uint32_t kNeg = float_order_key(neg_inf());
+  const int win = (int)min(max(a.derive_window, (int64_t)0), L);
+  const uint32_t bsz = (uint32_t)min(a.block_size, (int64_t)0x7fffffff);
+#pragma unroll
+  for (int it = 0; it < kRows; ++it) {
+    const int ql = wave * kRows + it;
+    const int64_t r = q0 + ql;
+    if (r >= L) break;  // uniform
+    // (32-bit: row and window are below 2^31)
+    const uint32_t lc = (uint32_t)max((int)r - win, 0) / bsz;
+    const uint32_t rc = (uint32_t)min((int)r + win, (int)L - 1) / bsz;
+    uint32_t key[kPer];
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+      const int c = lane + 64 * i;
+      const float m = mx_s[min(c, kC - 1) * kPitch + ql];
+      bool dropped = false;
+      if (a.derive_window >= 0)
+        dropped = ((uint32_t)c >= lc && (uint32_t)c <= rc) || cbad[min(c, kC - 1)] != 0;
+      else
+        dropped = (dropbits >> (kPer * it + i)) & 1u;
+      // 0 is below every real key: never picked
+      key[i] = c < C ? (dropped ? kNeg : float_order_key(m)) : 0u;
+    }
+    int16_t* plist = picks + ql * K;
+    if (lane < K) plist[lane] = -1;
+    const uint64_t sel = WaveSelect<kPer>::run(key, kPer, K);
+    int base = 0;
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+      const bool p = (sel >> i) & 1ull;
+      const uint64_t pb = __builtin_amdgcn_ballot_w64(p);
+      if (p) plist[base + __builtin_popcountll(pb & ((1ull << lane) - 1ull))] =
+          (int16_t)(lane + 64 * i);
+      base += __builtin_popcountll(pb);
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // this wave's list
+    if (lane < K) a.indices[((b * L + r) * a.Hkv + h) * K + lane] = plist[lane];
+  }
+  __syncthreads();
+  if (!scoring) return;
+
+  // ---- output ---------------------------------------------------------------
+  // Query j's chunk c at unit (c >> 2) ^ (j & 15) of its row (8-byte units: a
+  // tile's writes touch distinct banks).
+  uint16_t* raw = reinterpret_cast<uint16_t*>(smem + g * Lay::kRaw);
+  static_assert(kC % 64 == 0, "units come in blocks of 16");
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int u = 0; u < QT; ++u) {
+      u32x2_t w;
+      w[0] = pack_bf16x2(S[t][u][0] * a.sm_scale, S[t][u][1] * a.sm_scale);
+      w[1] = pack_bf16x2(S[t][u][2] * a.sm_scale, S[t][u][3] * a.sm_scale);
+      *reinterpret_cast<u32x2_t*>(raw + (16 * u + j) * kC + 4 * ((4 * t + grp) ^ j)) = w;
+    }
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // this wave's tile
+  auto raw_at = [&](int ql, int c) {
+    return c < 0 ? 0xff80u  // -inf past the picks
+                 : (uint32_t)raw[ql * kC + 4 * ((c >> 2) ^ (ql & 15)) + (c & 3)];
+  };
+  uint16_t* out = reinterpret_cast<uint16_t*>(a.scores);
+  const int nq = (int)min((int64_t)kQ, L - q0);
+  if (a.vec_out) {
+    const int k8 = K >> 3;
+    for (int e = lane; e < nq * k8; e += 64) {
+      const int ql = e / k8, s0 = 8 * (e - ql * k8);
+      const u32x4_t pk = *reinterpret_cast<const u32x4_t*>(picks + ql * K + s0);
+      u32x4_t o;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        o[i] = raw_at(ql, (int)(int16_t)(pk[i] & 0xffffu)) |
+               (raw_at(ql, (int)(int16_t)(pk[i] >> 16)) << 16);
+      *reinterpret_cast<u32x4_t*>(out + (((b * L + q0 + ql) * a.Hkv + h) * G + g) * K + s0) = o;
+    }
+  } else {
+    for (int e = lane; e < nq * K; e += 64) {
+      const int ql = e / K, s = e - ql * K;
+      out[(((b * L + q0 + ql) * a.Hkv + h) * G + g) * K + s] =
+          (uint16_t)raw_at(ql, picks[ql * K + s]);
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// One-pass path, 129 to 256 chunks and enough queries to fill the chip with
+// 128 of them per workgroup: every head in each wave.
 //
 // A workgroup takes 128 queries of one KV head, 16 per wave; a wave keeps
 // its queries' running max over heads M for all 256 chunks in registers.
@@ -119,22 +474,19 @@ __device__ __forceinline__ const uint16_t* lmk_row(const RouteArgs& a, int64_t b
 //           wave's [16][256] LDS tile, gathered at the picks.
 // One head's landmark keys sit in LDS while the next head's stream in.
 // ---------------------------------------------------------------------------
-constexpr int kFastThreads = 512;  // 8 waves x 16 queries
-constexpr int kFastQ = 128;        // queries per workgroup
-constexpr int kFastMaxTopk = 64;
-
-typedef __attribute__((address_space(3))) void lds_void_t;
+constexpr int kTileThreads = 512;  // 8 waves x 16 queries
+constexpr int kTileQ = 128;        // queries per workgroup
 
 // LDS carve-up.  Two landmark buffers ([256][128] bf16, 16-byte parts
 // XOR-swizzled: part p of row c at unit 16 c + (p ^ (c & 15))); in pass 2
 // the one pass 1 ends off holds the waves' raw-logit tiles.  Two bias rows
 // (-inf past C), the chunk flags and the pick lists [128][K] int16.
-struct FastLayout {
+struct TileLayout {
   static constexpr size_t lmk = 0;                    // [2][256][128] bf16
   static constexpr size_t bias = 2 * 256 * 128 * 2;   // [2][256] f32
   static constexpr size_t cbad = bias + 2 * 256 * 4;  // [256] u8
   static constexpr size_t picks = cbad + 256;         // [128][K] i16
-  static size_t total(int K) { return picks + (size_t)kFastQ * K * 2; }
+  static size_t total(int K) { return picks + (size_t)kTileQ * K * 2; }
 };
 
 __device__ __forceinline__ int across4_sum_i(int v) {
@@ -172,14 +524,14 @@ __device__ __forceinline__ int chunk_rank(const uint64_t (&m)[4], int grp, int t
 }
 
 template <int G>
-__global__ void __launch_bounds__(kFastThreads, 1) route_topk_fast_kernel(RouteArgs a) {
+__global__ void __launch_bounds__(kTileThreads, 1) route_tile_kernel(RouteArgs a) {
   extern __shared__ __align__(16) unsigned char smem[];
   const int K = a.K;
-  float* bias_s = reinterpret_cast<float*>(smem + FastLayout::bias);
-  unsigned char* cbad = smem + FastLayout::cbad;
-  int16_t* picks = reinterpret_cast<int16_t*>(smem + FastLayout::picks);
+  float* bias_s = reinterpret_cast<float*>(smem + TileLayout::bias);
+  unsigned char* cbad = smem + TileLayout::cbad;
+  int16_t* picks = reinterpret_cast<int16_t*>(smem + TileLayout::picks);
   auto lmk_buf = [&](int i) {
-    return reinterpret_cast<uint16_t*>(smem + FastLayout::lmk) + i * 256 * 128;
+    return reinterpret_cast<uint16_t*>(smem + TileLayout::lmk) + i * 256 * 128;
   };
 
   const int tid = threadIdx.x;
@@ -188,7 +540,7 @@ __global__ void __launch_bounds__(kFastThreads, 1) route_topk_fast_kernel(RouteA
   const int64_t b = blockIdx.z;
   const int h = blockIdx.y;
   const int64_t L = a.L, C = a.C;
-  const int64_t q0 = (int64_t)blockIdx.x * kFastQ;
+  const int64_t q0 = (int64_t)blockIdx.x * kTileQ;
   const int ql = 16 * wave + j;            // this lane's query within the workgroup
   const int64_t r = q0 + ql;
   const bool rvalid = r < L;
@@ -197,25 +549,11 @@ __global__ void __launch_bounds__(kFastThreads, 1) route_topk_fast_kernel(RouteA
 
   // Chunks with no valid real key (the last slot of a chunk is its landmark).
   if (a.derive_window >= 0) {
-    for (int c = tid; c < 256; c += kFastThreads) {
+    for (int c = tid; c < 256; c += kTileThreads) {
       bool any = false;
       if (c < C) {
         if (a.key_valid) {
-          const uint8_t* kv = a.key_valid + b * L + (int64_t)c * a.block_size;
-          if (a.block_size == 64 && ((uintptr_t)kv & 15) == 0) {
-            u32x4_t acc = {0u, 0u, 0u, 0u};
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-              const u32x4_t x = *reinterpret_cast<const u32x4_t*>(kv + 16 * v);
-              acc[0] |= x[0];
-              acc[1] |= x[1];
-              acc[2] |= x[2];
-              acc[3] |= v == 3 ? (x[3] & 0x00ffffffu) : x[3];
-            }
-            any = (acc[0] | acc[1] | acc[2] | acc[3]) != 0u;
-          } else {
-            for (int64_t s = 0; s < a.block_size - 1; ++s) any |= kv[s] != 0;
-          }
+          any = chunk_has_valid_key(a.key_valid + b * L + (int64_t)c * a.block_size, a.block_size);
         } else {
           any = a.block_size > 1;
         }
@@ -347,15 +685,7 @@ __global__ void __launch_bounds__(kFastThreads, 1) route_topk_fast_kernel(RouteA
     }
     const float s2 = across4_sum(sm);
     const float lse2 = m2 == neg_inf() ? neg_inf() : m2 + log2_hw(s2);
-    float tot = 0.f;
-    if (!a.pre_softmax) {
-      // logaddexp(local LSE, LSE) in base 2, back to natural units.  A -inf
-      // total (no visible logit at all) is clamped to -FLT_MAX: finite x - tot
-      // then ties at the top like x - (-inf) = +inf would, and -inf stays.
-      const float lv2 = lse_c * kLog2e;
-      const float hi = fmaxf(lv2, lse2), lo = fminf(lv2, lse2);
-      tot = hi == neg_inf() ? -__FLT_MAX__ : (hi + log2_hw(1.f + exp2_hw(lo - hi))) * kLn2;
-    }
+    const float tot = a.pre_softmax ? 0.f : route_total(lse_c, lse2);
 #pragma unroll
     for (int t = 0; t < 16; ++t)
 #pragma unroll
@@ -513,10 +843,10 @@ __global__ void __launch_bounds__(kFastThreads, 1) route_topk_fast_kernel(RouteA
   // operations in order).
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   int32_t* irow = a.indices + ((b * L + r) * a.Hkv + h) * K;
-  // Output slots: with vec_out a lane writes the K / 4 consecutive slots
+  // Output slots: with vec32_out a lane writes the K / 4 consecutive slots
   // s0 .. s0 + K / 4 - 1 of its query (one 16-byte store per 8 scores, per
   // 4 indices), its picks held as int16 pairs in pk; else slots grp + 4 i.
-  const bool vec = a.vec_out != 0;
+  const bool vec = a.vec32_out != 0;
   const int per = K >> 2, nv = K >> 5, s0 = per * grp;
   uint32_t pk[8];
 #pragma unroll
@@ -617,6 +947,465 @@ __global__ void __launch_bounds__(kFastThreads, 1) route_topk_fast_kernel(RouteA
     }
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks) Qc[ks] = Qn[ks];
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Scan path, for many rows against more chunks than the one-pass path holds:
+// the selection scores [B, L, Hkv, Cp] (fp32, Cp = C rounded up to 16) pass
+// through the workspace, a seventh of the raw logits.  Three kernels:
+//
+// route_lse_kernel: a workgroup of 8 waves holds one head of 128 queries, 16
+// per wave, and forms their logaddexp(local LSE, LSE over all chunks).
+// route_scan_kernel: a workgroup of 8 waves holds 128 queries of one KV head,
+// 16 per wave with every head's Q operand in registers, and forms the maximum
+// over heads of x - that total, dropped chunks -inf.
+// route_pick_kernel: a wave per row picks its K largest and forms the picks'
+// raw logits again.
+//
+// Landmark rows stream through an LDS ring in both scans, filled by DMA.  The
+// products are S = q . lmk^T: lane (j, grp) holds chunk 16 t + j for queries
+// 4 grp + i.  A row's LSE is summed as the workgroup selection's wave form
+// sums it -- chunks c mod 64 in running (max, sum) pairs, then a butterfly over
+// the 64 -- here 4 pairs per lane and query, so that near ties between heads
+// fall the same way as they always did.
+//
+// Measured at 65536 queries x 4 KV heads x 7 heads against 1024 chunks: 1640
+// (LSE) + 1170 (scan) + 1440 (pick) us; 7590 + 6260 us with the fp32 logits of
+// every head through memory (7.5 GB written and read).  The LSE kernel is bound
+// by the ~25 VALU instructions of each term, the scan by its products and
+// their 7-head epilogue at two waves per SIMD, the pick by the gather.
+// ---------------------------------------------------------------------------
+constexpr int kScanThreads = 512;
+constexpr int kScanQ = 128;
+constexpr int kScanRing = 4;
+constexpr int kLseRing = 3;  // 64-chunk stages of one head
+constexpr int kPickRing = 2;
+constexpr int kScanMaxChunks = 4096;
+
+inline int64_t scan_chunks(int64_t chunks) { return (chunks + 15) / 16 * 16; }
+
+// The scaled logit plus the bias, each rounded (no fused multiply-add).
+__device__ __forceinline__ float scaled_plus(float acc, float scale, float bias) {
+#pragma clang fp contract(off)
+  const float s = acc * scale;
+  return s + bias;
+}
+
+// The causal limit of row r as a chunk count in [0, C].
+__device__ __forceinline__ int chunk_limit(const RouteArgs& a, int64_t r) {
+  return (int)(a.is_causal ? max((int64_t)0, min(a.C, causal_limit(a, r))) : a.C);
+}
+
+__global__ void __launch_bounds__(kScanThreads, 4)
+    route_lse_kernel(RouteArgs a, float* __restrict__ total) {
+  __shared__ __align__(16) unsigned char ring[kLseRing][64 * 256];
+  __shared__ float bias_s[kLseRing][64];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int j = lane & 15, grp = lane >> 4;
+  const int G = a.G;
+  const int64_t b = blockIdx.z;
+  const int h = blockIdx.y / G, g = blockIdx.y - h * G;
+  const int64_t L = a.L;
+  const int C = (int)a.C;
+  const int ns = (C + 63) >> 6;  // stages
+  const int64_t r0 = (int64_t)blockIdx.x * kScanQ + 16 * wave;
+  u32x4_t Q[4];
+  {
+    const int64_t row = ((b * L + min(r0 + j, L - 1)) * a.Hkv + h) * G + g;
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks)
+      Q[ks] = *reinterpret_cast<const u32x4_t*>(a.q + row * 128 + 8 * grp + 32 * ks);
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) asm volatile("" : "+v"(Q[ks]));  // before any DMA
+  }
+  // Stage s: 64 chunks' rows, 2 of the 16 DMA instructions per wave (4 rows of
+  // 256 bytes each; part p of row r at unit p ^ (r & 15)), and with a bias its
+  // 64 values (every wave issues it: the same bytes, the same count of loads).
+  const uint32_t rowlen = (uint32_t)(a.per_head_lmk ? a.Hkv * G : a.Hkv) * 128u;
+  const uint32_t head = 256u * (uint32_t)(a.per_head_lmk ? h * G + g : h);
+  const __amdgpu_buffer_rsrc_t lrs = lmk_rsrc(a, b, rowlen);
+  const uint32_t blen = (uint32_t)(a.Hkv * G);
+  const __amdgpu_buffer_rsrc_t brs = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<float*>(a.bias ? a.bias + b * C * (int64_t)blen : a.lse), (short)0,
+      a.bias ? (int)((uint32_t)C * blen * 4u) : 0, 0x00020000);
+  if (!a.bias && tid < 64)
+    for (int s = 0; s < kLseRing; ++s) bias_s[s][tid] = 0.f;
+  auto stage = [&](int s) {
+    const int slot = s % kLseRing;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int n = 2 * wave + i, row = 4 * n + grp;
+      const uint32_t c = (uint32_t)min(64 * s + row, C - 1);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          lrs, (lds_void_t*)(ring[slot] + n * 1024), 16,
+          2u * (__umul24(c, rowlen) + 8u * (uint32_t)(j ^ (row & 15))), head, 0, 0);
+    }
+    if (a.bias) {  // uniform
+      const uint32_t c = (uint32_t)min(64 * s + lane, C - 1);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(brs, (lds_void_t*)bias_s[slot], 4,
+                                               4u * __umul24(c, blen), 4u * (uint32_t)(h * G + g),
+                                               0, 0);
+    }
+  };
+  for (int s = 0; s < kLseRing - 1 && s < ns; ++s) stage(s);
+  int climit[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) climit[i] = chunk_limit(a, min(r0 + 4 * grp + i, L - 1));
+  // The pair of (query 4 grp + i, chunks with c mod 64 = 16 k + j).
+  float m[4][4], sum[4][4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      m[k][i] = neg_inf();
+      sum[k][i] = 0.f;
+    }
+  auto step = [&](int s, bool hide) {
+    // one stage may be in flight behind the awaited one
+    if (s + 1 < ns) {
+      if (a.bias) asm volatile("s_waitcnt vmcnt(3)" ::: "memory");
+      else asm volatile("s_waitcnt vmcnt(2)" ::: "memory");
+    } else {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (s + kLseRing - 1 < ns) stage(s + kLseRing - 1);
+    const int slot = s % kLseRing;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const unsigned char* brow = ring[slot] + (16 * k + j) * 256;
+      f32x4_t x = zero4();
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks)
+        x = mfma_bf16_16x16x32(
+            Q[ks], *reinterpret_cast<const u32x4_t*>(brow + (((4 * ks + grp) ^ j) * 16)), x);
+      const float bv = bias_s[slot][16 * k + j];
+      const int c = 64 * s + 16 * k + j;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        float v = scaled_plus(x[i], a.sm_scale, bv);
+        if (hide && c >= climit[i]) v = neg_inf();
+        // a new max scales the sum so far: sum e + 1, else sum + e, with
+        // e = exp(-|v - max|), one rounding each
+        const bool up = v > m[k][i];
+        float e = expf(-fabsf(v - m[k][i]));
+        e = v == neg_inf() ? 0.f : e;
+        sum[k][i] = __builtin_fmaf(up ? sum[k][i] : 1.f, e, up ? 1.f : sum[k][i]);
+        m[k][i] = fmaxf(m[k][i], v);
+      }
+    }
+  };
+  const int whole = a.is_causal ? 0 : C >> 6;
+  for (int s = 0; s < whole; ++s) step(s, false);
+  for (int s = whole; s < ns; ++s) step(s, true);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    // over the 64 pairs: j by lane moves (1, 2, 4, 8), then k (16, 32)
+    float mm = fmaxf(fmaxf(m[0][i], m[1][i]), fmaxf(m[2][i], m[3][i]));
+#pragma unroll
+    for (int o = 1; o < 16; o <<= 1) mm = fmaxf(mm, __shfl_xor(mm, o, 64));
+    float ss[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      ss[k] = m[k][i] == neg_inf() ? 0.f : sum[k][i] * expf(m[k][i] - mm);
+#pragma unroll
+      for (int o = 1; o < 16; o <<= 1) ss[k] += __shfl_xor(ss[k], o, 64);
+    }
+    const float st = (ss[0] + ss[1]) + (ss[2] + ss[3]);
+    const float lse_h = mm == neg_inf() ? mm : mm + logf(st);
+    const int64_t r = r0 + 4 * grp + i;
+    if (j == 0 && r < L) {
+      const int64_t at = ((b * L + r) * a.Hkv + h) * G + g;
+      total[at] = logaddexp_f(a.lse[at], lse_h);
+    }
+  }
+}
+
+template <int G>
+struct ScanLayout {
+  static constexpr int kTile = 16 * G * 256;             // a tile's landmark rows
+  static constexpr int kBias = kScanRing * kTile;        // [ring][8][16] f32
+  static constexpr int kBad = kBias + kScanRing * 512;   // [Cp / 64] u64
+  static constexpr int kTotal = kBad + kScanMaxChunks / 8;
+};
+
+// total: [B, L, Hkv, G], or null (pre-softmax selection).
+template <int G>
+__global__ void __launch_bounds__(kScanThreads, 2)
+    route_scan_kernel(RouteArgs a, const float* __restrict__ total, float* __restrict__ best,
+                      int Cp) {
+  using Lay = ScanLayout<G>;
+  extern __shared__ __align__(16) unsigned char smem[];
+  float* bias_s = reinterpret_cast<float*>(smem + Lay::kBias);
+  uint64_t* bad_s = reinterpret_cast<uint64_t*>(smem + Lay::kBad);
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int j = lane & 15, grp = lane >> 4;
+  const int64_t b = blockIdx.z;
+  const int h = blockIdx.y;
+  const int64_t L = a.L;
+  const int C = (int)a.C;
+  const int nt = Cp >> 4;
+  const int64_t r0 = (int64_t)blockIdx.x * kScanQ + 16 * wave;
+
+  // Chunks with no valid real key, as bits.
+  if (a.derive_window >= 0)
+    for (int c0 = 64 * wave; c0 < Cp; c0 += kScanThreads) {
+      const int c = c0 + lane;
+      bool any = c < C && a.block_size > 1;
+      if (any && a.key_valid)
+        any = chunk_has_valid_key(a.key_valid + b * L + (int64_t)c * a.block_size, a.block_size);
+      const uint64_t m = __builtin_amdgcn_ballot_w64(!any);
+      if (lane == 0) bad_s[c0 >> 6] = m;
+    }
+  // Q rows r0 + j of every head; the totals of queries r0 + 4 grp + i (rows
+  // past L re-read row L - 1).
+  u32x4_t Q[G][4];
+  float tot[G][4];
+  {
+    const int64_t row = ((b * L + min(r0 + j, L - 1)) * a.Hkv + h) * G;
+#pragma unroll
+    for (int g = 0; g < G; ++g)
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks)
+        Q[g][ks] =
+            *reinterpret_cast<const u32x4_t*>(a.q + (row + g) * 128 + 8 * grp + 32 * ks);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int64_t at = ((b * L + min(r0 + 4 * grp + i, L - 1)) * a.Hkv + h) * G;
+#pragma unroll
+      for (int g = 0; g < G; ++g) tot[g][i] = total ? total[at + g] : 0.f;
+    }
+#pragma unroll
+    for (int g = 0; g < G; ++g)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        asm volatile("" : "+v"(Q[g][i]));  // before any DMA
+        asm volatile("" : "+v"(tot[g][i]));
+      }
+  }
+  // Tile t into slot t % kScanRing: 4 DMA instructions of 4 rows x 256 bytes
+  // per head (part p of row r at unit p ^ r; rows >= C re-read row C - 1) and,
+  // with a bias, 2 of 64 floats for its [G][16] values, dealt to the waves in
+  // turn.  Waves past the last one repeat it (the same bytes), so that every
+  // wave counts the same number of loads in flight.
+  const uint32_t rowlen = (uint32_t)(a.per_head_lmk ? a.Hkv * G : a.Hkv) * 128u;
+  const __amdgpu_buffer_rsrc_t lrs = lmk_rsrc(a, b, rowlen);
+  const uint32_t blen = (uint32_t)(a.Hkv * G);
+  const __amdgpu_buffer_rsrc_t brs = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<float*>(a.bias ? a.bias + b * C * (int64_t)blen : a.lse), (short)0,
+      a.bias ? (int)((uint32_t)C * blen * 4u) : 0, 0x00020000);
+  constexpr int kRows = 4 * G;
+  constexpr int kMine = (kRows + 2 + 7) / 8;  // instructions per wave and tile
+  const int ninstr = kRows + (a.bias ? 2 : 0);
+  auto stage = [&](int t) {
+    const int slot = t % kScanRing;
+#pragma unroll
+    for (int i = 0; i < kMine; ++i) {
+      const int n = min(wave + 8 * i, ninstr - 1);
+      if (n < kRows) {  // uniform
+        const int row = 4 * (n & 3) + grp;
+        const uint32_t c = (uint32_t)min(16 * t + row, C - 1);
+        const uint32_t head = 256u * (uint32_t)(a.per_head_lmk ? h * G + (n >> 2) : h);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(
+            lrs, (lds_void_t*)(smem + slot * Lay::kTile + n * 1024), 16,
+            2u * (__umul24(c, rowlen) + 8u * (uint32_t)(j ^ row)), head, 0, 0);
+      } else {
+        const int e = 64 * (n - kRows) + lane;
+        const uint32_t c = (uint32_t)min(16 * t + (e & 15), C - 1);
+        const uint32_t g = (uint32_t)min(e >> 4, G - 1);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(
+            brs, (lds_void_t*)(smem + Lay::kBias + slot * 512 + 256 * (n - kRows)), 4,
+            4u * (__umul24(c, blen) + g), 4u * (uint32_t)(h * G), 0, 0);
+      }
+    }
+  };
+  if (!a.bias) {
+    for (int i = tid; i < kScanRing * 128; i += kScanThreads) bias_s[i] = 0.f;
+  }
+#pragma unroll
+  for (int t = 0; t < kScanRing - 1; ++t)
+    if (t < nt) stage(t);
+  int climit[4], lc[4], rc[4];
+  const int win = (int)min(max(a.derive_window, (int64_t)0), L);
+  const uint32_t bsz = (uint32_t)min(a.block_size, (int64_t)0x7fffffff);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int64_t r = min(r0 + 4 * grp + i, L - 1);
+    climit[i] = chunk_limit(a, r);
+    lc[i] = (int)((uint32_t)max((int)r - win, 0) / bsz);
+    rc[i] = (int)((uint32_t)min((int)r + win, (int)L - 1) / bsz);
+  }
+  auto step = [&](int t, bool hide) {
+    // Tile t is in LDS for every wave once each has waited for its own share;
+    // the barrier also frees slot t - 1 for tile t + ring - 1.
+    const int later = min(kScanRing - 2, nt - 1 - t);
+    if (later >= 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * kMine) : "memory");
+    else if (later == 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kMine) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (t + kScanRing - 1 < nt) stage(t + kScanRing - 1);
+    const int slot = t % kScanRing;
+    const unsigned char* tile = smem + slot * Lay::kTile + j * 256;
+    // the products of all heads first, so that their chains overlap
+    f32x4_t x[G];
+#pragma unroll
+    for (int g = 0; g < G; ++g) x[g] = zero4();
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks)
+#pragma unroll
+      for (int g = 0; g < G; ++g)
+        x[g] = mfma_bf16_16x16x32(Q[g][ks],
+                                  *reinterpret_cast<const u32x4_t*>(
+                                      tile + g * 4096 + (((4 * ks + grp) ^ j) * 16)),
+                                  x[g]);
+    float y[4] = {neg_inf(), neg_inf(), neg_inf(), neg_inf()};
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      const float bv = bias_s[slot * 128 + 16 * g + j];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        // (an x of -inf stays -inf beside an infinite total)
+        const float v = scaled_plus(x[g][i], a.sm_scale, bv);
+        y[i] = fmaxf(y[i], v == neg_inf() ? v : v - tot[g][i]);
+      }
+    }
+    const int c = 16 * t + j;
+    const bool bad = a.derive_window >= 0 && ((bad_s[t >> 2] >> (16 * (t & 3) + j)) & 1ull);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int64_t r = r0 + 4 * grp + i;
+      if (hide && c >= climit[i]) y[i] = neg_inf();
+      if (a.derive_window >= 0) {  // uniform
+        if (bad | ((c >= lc[i]) & (c <= rc[i]))) y[i] = neg_inf();
+      } else if (a.drop) {
+        if (a.drop[(b * L + min(r, L - 1)) * C + min(c, C - 1)] != 0) y[i] = neg_inf();
+      }
+      if (r < L) best[((b * L + r) * a.Hkv + h) * Cp + c] = y[i];
+    }
+  };
+  const int whole = a.is_causal ? 0 : C >> 4;
+  for (int t = 0; t < whole; ++t) step(t, false);
+  for (int t = whole; t < nt; ++t) step(t, true);
+}
+
+template <int G, int PER>
+__global__ void __launch_bounds__(256)
+    route_pick_kernel(RouteArgs a, const float* __restrict__ best, int Cp) {
+  __shared__ int32_t list_s[4][64];
+  __shared__ __align__(16) unsigned char ring_s[4][kPickRing * 4096];
+  __shared__ __align__(16) unsigned char q_s[4][2048];
+  const int lane = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int j = lane & 15, grp = lane >> 4;
+  const int64_t r = (int64_t)blockIdx.x * 4 + wv;
+  if (r >= a.L) return;  // wave-uniform
+  const int h = blockIdx.y;
+  const int64_t b = blockIdx.z;
+  const int C = (int)a.C, K = a.K;
+  const int n = (C + 63) >> 6;  // <= PER
+  const int64_t row = (b * a.L + r) * a.Hkv + h;
+  // The row's G query heads to LDS (past them: zeros).
+  {
+    const __amdgpu_buffer_rsrc_t qrs = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint16_t*>(a.q + row * G * 128), (short)0, G * 256, 0x00020000);
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(qrs, (lds_void_t*)(q_s[wv] + 1024 * i), 16,
+                                               16u * lane, 1024u * i, 0, 0);
+  }
+  // The loads are unconditional (slots past the row read its last score), all
+  // in flight together.
+  uint32_t key[PER];
+  {
+    float v[PER];
+#pragma unroll
+    for (int i = 0; i < PER; ++i) v[i] = best[row * Cp + min(lane + 64 * i, C - 1)];
+#pragma unroll
+    for (int i = 0; i < PER; ++i)
+      key[i] = lane + 64 * i < C ? float_order_key(v[i]) : 0u;  // 0: never picked
+  }
+  const uint64_t sel = WaveSelect<PER>::run(key, n, K);
+  int32_t* list = list_s[wv];
+  int total = 0;
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    if (i >= n) continue;  // uniform
+    const bool p = (sel >> i) & 1ull;
+    const uint64_t pb = __builtin_amdgcn_ballot_w64(p);
+    if (p) list[total + __builtin_popcountll(pb & ((1ull << lane) - 1ull))] = lane + 64 * i;
+    total += __builtin_popcountll(pb);
+  }
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // this wave's list only
+  if (lane < K) a.indices[row * K + lane] = lane < total ? list[lane] : -1;
+  // Raw logits of the picks for every head: item (T, g) is a product whose
+  // rows are picks 16 T .. 16 T + 15's landmark rows of head g and whose
+  // every column is the query.  The rows pass through the wave's LDS ring, by
+  // DMA in whole 256-byte rows (part p of row r at unit p ^ r; operand-shaped
+  // loads would touch 16 rows per 16 bytes of each: 2.29 ms at 262144 rows of
+  // 1024 chunks).  Lanes with j = g keep head g's picks 16 T + 4 grp + i.
+  const uint32_t rowlen = (uint32_t)(a.per_head_lmk ? a.Hkv * G : a.Hkv) * 128u;
+  const __amdgpu_buffer_rsrc_t lrs = lmk_rsrc(a, b, rowlen);
+  unsigned char* ring = ring_s[wv];
+  const int items = (K + 15) / 16 * G;
+  auto stage = [&](int it) {
+    const int T = it / G, g = it - T * G;
+    const uint32_t head = 256u * (uint32_t)(a.per_head_lmk ? h * G + g : h);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int rr = 4 * k + grp, p = 16 * T + rr;
+      const uint32_t c = p < total ? (uint32_t)list[p] : 0u;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          lrs, (lds_void_t*)(ring + (it % kPickRing) * 4096 + 1024 * k), 16,
+          2u * (__umul24(c, rowlen) + 8u * (uint32_t)(j ^ rr)), head, 0, 0);
+    }
+  };
+  for (int it = 0; it < kPickRing && it < items; ++it) stage(it);
+  for (int T = 0; 16 * T < K; ++T) {
+    f32x4_t keep = zero4();
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      const int it = T * G + g;
+      if (it + 1 < items) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+      else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      const unsigned char* arow = ring + (it % kPickRing) * 4096 + j * 256;
+      f32x4_t acc = zero4();
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks)
+        acc = mfma_bf16_16x16x32(
+            *reinterpret_cast<const u32x4_t*>(arow + (((4 * ks + grp) ^ j) * 16)),
+            *reinterpret_cast<const u32x4_t*>(q_s[wv] + 256 * g + 64 * ks + 16 * grp), acc);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) keep[i] = j == g ? acc[i] : keep[i];
+      if (it + kPickRing < items) {
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the slot has been read
+        stage(it + kPickRing);
+      }
+    }
+    const int s0 = 16 * T + 4 * grp;
+    if (j < G) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) keep[i] = s0 + i < total ? keep[i] * a.sm_scale : neg_inf();
+      const int64_t at = (row * G + j) * K + s0;
+      if (a.scores_fp32) {
+        for (int i = 0; i < 4; ++i)
+          if (s0 + i < K) reinterpret_cast<float*>(a.scores)[at + i] = keep[i];
+      } else if (a.vec_out) {  // K % 8 == 0: whole 8-byte groups
+        if (s0 < K)
+          *reinterpret_cast<u32x2_t*>(reinterpret_cast<uint16_t*>(a.scores) + at) =
+              u32x2_t{pack_bf16x2(keep[0], keep[1]), pack_bf16x2(keep[2], keep[3])};
+      } else {
+        for (int i = 0; i < 4; ++i)
+          if (s0 + i < K)
+            reinterpret_cast<uint16_t*>(a.scores)[at + i] = (uint16_t)f32_to_bf16(keep[i]);
+      }
+    }
   }
 }
 
@@ -1245,186 +2034,6 @@ __global__ void __launch_bounds__(kSelThreads) route_select_kernel(RouteArgs a,
   }
 }
 
-// Selection with one wave per (row, KV head, batch) and no barrier, for long
-// sequences (many rows): chunk c = lane + 64 i, so the wave selection's order
-// index is the chunk index and ties still go to the lower chunk.  The head
-// LSEs come from one pass with a per-lane online max / sum; the keys are
-// formed from the logits held in registers when PER * G <= 128 (C <= 1024 at
-// G = 8) and from a second read of the row otherwise.  Same score, LSE, drop
-// and tie rules as route_select_kernel.  Global loads are unconditional
-// (slots past the row read chunk 0) and issued kB slots at a time with no
-// branch between them: loads inside per-slot branches were each waited for
-// at the branch's end.  topk <= 64: the picks' chunks pass through the
-// wave's LDS row so that lane t writes output slot t.
-template <int G, int PER>
-__global__ void __launch_bounds__(256) route_select_wave_kernel(RouteArgs a,
-                                                                const float* __restrict__ raw) {
-  constexpr bool kHold = PER * G <= 128;
-  constexpr int kB = kHold ? PER : 8;  // slots per batch of loads
-  __shared__ int32_t pick_c[4][64];
-  const int64_t C = a.C, L = a.L;
-  const int K = a.K;
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int64_t r = (int64_t)blockIdx.x * 4 + wv;
-  if (r >= L) return;  // wave-uniform
-  const int h = blockIdx.y;
-  const int64_t b = blockIdx.z;
-  const int n = (int)((C + 63) / 64);  // <= PER
-  const int64_t row = (b * L + r) * a.Hkv + h;
-  const float* xr = raw + row * (int64_t)G * C;
-  const int64_t climit = a.is_causal ? causal_limit(a, r) : C;
-  const float* bias = a.bias ? a.bias + (b * C * a.Hkv + h) * G : nullptr;  // + c * Hkv * G + g
-  const int64_t bstride = (int64_t)a.Hkv * G;
-
-  // x of slots i0 .. i0 + kB - 1: raw + bias, -inf past the row or the
-  // causal limit.
-  auto load_batch = [&](int i0, float (&v)[kB][G]) {
-#pragma unroll
-    for (int ii = 0; ii < kB; ++ii) {
-      const int64_t c = lane + 64 * (int64_t)(i0 + ii);
-      const int64_t cc = i0 + ii < n && c < C ? c : 0;
-#pragma unroll
-      for (int g = 0; g < G; ++g) v[ii][g] = xr[(int64_t)g * C + cc];
-    }
-    if (bias) {
-#pragma unroll
-      for (int ii = 0; ii < kB; ++ii) {
-        const int64_t c = lane + 64 * (int64_t)(i0 + ii);
-        const int64_t cc = i0 + ii < n && c < C ? c : 0;
-#pragma unroll
-        for (int g = 0; g < G; ++g) v[ii][g] += bias[cc * bstride + g];
-      }
-    }
-#pragma unroll
-    for (int ii = 0; ii < kB; ++ii) {
-      const int64_t c = lane + 64 * (int64_t)(i0 + ii);
-      const bool ok = i0 + ii < n && c < C && c < climit;
-#pragma unroll
-      for (int g = 0; g < G; ++g) v[ii][g] = ok ? v[ii][g] : neg_inf();
-    }
-  };
-
-  float hold[kB][G];
-  float m[G], sum[G];
-#pragma unroll
-  for (int g = 0; g < G; ++g) {
-    m[g] = neg_inf();
-    sum[g] = 0.f;
-  }
-#pragma unroll
-  for (int i0 = 0; i0 < PER; i0 += kB) {
-    if (i0 >= n) break;  // uniform
-    load_batch(i0, hold);
-#pragma unroll
-    for (int ii = 0; ii < kB; ++ii)
-#pragma unroll
-      for (int g = 0; g < G; ++g) {
-        const float v = hold[ii][g];
-        if (v > m[g]) {
-          sum[g] = (m[g] == neg_inf() ? 0.f : sum[g] * expf(m[g] - v)) + 1.f;
-          m[g] = v;
-        } else if (v != neg_inf()) {
-          sum[g] += expf(v - m[g]);
-        }
-      }
-  }
-  float tot[G];
-#pragma unroll
-  for (int g = 0; g < G; ++g) {
-    const float mm = wave_max(m[g]);
-    const float ss = wave_sum(m[g] == neg_inf() ? 0.f : sum[g] * expf(m[g] - mm));
-    const float lse_h = mm == neg_inf() ? mm : mm + logf(ss);
-    tot[g] = a.pre_softmax ? 0.f : logaddexp_f(a.lse[row * G + g], lse_h);
-  }
-
-  // Drop flags (bit i: slot i), one uniform branch per drop source.
-  uint64_t dropbits = 0ull;
-  if (a.derive_window >= 0) {
-    const int64_t lc = max(r - a.derive_window, (int64_t)0) / a.block_size;
-    const int64_t rc = min(r + a.derive_window, L - 1) / a.block_size;
-#pragma unroll
-    for (int i = 0; i < PER; ++i) {
-      const int64_t c = lane + 64 * (int64_t)i;
-      const int64_t cc = i < n && c < C ? c : 0;
-      bool any = a.block_size > 1;
-      if (a.key_valid) any = chunk_has_valid_key(a.key_valid + b * L + cc * a.block_size,
-                                                 a.block_size);
-      dropbits |= (uint64_t)((c >= lc && c <= rc) || !any) << i;
-    }
-  } else if (a.drop) {
-    const int32_t* drow = a.drop + (b * L + r) * C;
-#pragma unroll
-    for (int i = 0; i < PER; ++i) {
-      const int64_t c = lane + 64 * (int64_t)i;
-      dropbits |= (uint64_t)(drow[i < n && c < C ? c : 0] != 0) << i;
-    }
-  }
-  uint32_t key[PER];
-#pragma unroll
-  for (int i0 = 0; i0 < PER; i0 += kB) {
-    if (!kHold && i0 < n) load_batch(i0, hold);  // uniform
-#pragma unroll
-    for (int ii = 0; ii < kB; ++ii) {
-      const int i = i0 + ii;
-      const int64_t c = lane + 64 * (int64_t)i;
-      float best = neg_inf();
-#pragma unroll
-      for (int g = 0; g < G; ++g) {
-        const float x = hold[ii][g];
-        best = fmaxf(best, x == neg_inf() ? x : x - tot[g]);
-      }
-      // 0 is below every real key: never picked
-      key[i] = i < n && c < C ? float_order_key(((dropbits >> i) & 1ull) ? neg_inf() : best) : 0u;
-    }
-  }
-
-  const uint64_t picks = WaveSelect<PER>::run(key, n, K);
-  const uint64_t below = (1ull << lane) - 1ull;
-  int base = 0;
-#pragma unroll
-  for (int i = 0; i < PER; ++i) {
-    if (i >= n) continue;  // uniform
-    const bool p = (picks >> i) & 1ull;
-    const uint64_t pb = __builtin_amdgcn_ballot_w64(p);
-    if (p) pick_c[wv][base + __builtin_popcountll(pb & below)] = (int32_t)(lane + 64 * i);
-    base += __builtin_popcountll(pb);
-  }
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // this wave's LDS row only
-  // lane t writes output slot t (K <= 64)
-  if (lane < K) {
-    const int t = lane;
-    const bool live = t < base;
-    const int32_t c = live ? pick_c[wv][t] : 0;
-    float v[G];
-#pragma unroll
-    for (int g = 0; g < G; ++g) v[g] = xr[(int64_t)g * C + c];
-    a.indices[row * K + t] = live ? c : -1;
-#pragma unroll
-    for (int g = 0; g < G; ++g) {
-      if (a.scores_fp32)
-        reinterpret_cast<float*>(a.scores)[(row * G + g) * K + t] = live ? v[g] : neg_inf();
-      else
-        reinterpret_cast<uint16_t*>(a.scores)[(row * G + g) * K + t] =
-            live ? (uint16_t)f32_to_bf16(v[g]) : (uint16_t)0xff80u;
-    }
-  }
-}
-
-// Rows (token, KV head, batch) above which the wave selection replaces the
-// workgroup selection: below it a workgroup per row spreads a short block's
-// few rows over more of the chip.
-constexpr int64_t kWaveSelectRows = 4096;
-
-template <int G>
-int launch_select_wave(const RouteArgs& a, const float* raw, hipStream_t s) {
-  dim3 grid((unsigned)((a.L + 3) / 4), (unsigned)a.Hkv, (unsigned)a.B);
-  if (a.C <= 1024)
-    hipLaunchKernelGGL((route_select_wave_kernel<G, 16>), grid, dim3(256), 0, s, a, raw);
-  else
-    hipLaunchKernelGGL((route_select_wave_kernel<G, 64>), grid, dim3(256), 0, s, a, raw);
-  return mrsa_launch_status();
-}
-
 template <int G>
 int launch_select(const RouteArgs& a, const float* raw, hipStream_t s) {
   dim3 g2((unsigned)a.L, (unsigned)a.Hkv, (unsigned)a.B);
@@ -1438,11 +2047,6 @@ int launch_block(const RouteArgs& a, float* raw, hipStream_t s) {
   hipLaunchKernelGGL(route_logits_kernel, g1, dim3(64 * a.G), 0, s, a, raw);
   int st = mrsa_launch_status();
   if (st != MRSA_OK) return st;
-  if (a.B * a.L * a.Hkv >= kWaveSelectRows && a.C <= 4096 && a.K <= 64 &&
-      a.L <= 0x7ffffffc) {
-    if (a.G == 7) return launch_select_wave<7>(a, raw, s);
-    if (a.G == 8) return launch_select_wave<8>(a, raw, s);
-  }
   switch (a.G) {
     case 1: return launch_select<1>(a, raw, s);
     case 2: return launch_select<2>(a, raw, s);
@@ -1455,18 +2059,99 @@ int launch_block(const RouteArgs& a, float* raw, hipStream_t s) {
   }
 }
 
-// raw_ws: bf16 [B][L][Hkv][G][C] raw-score workspace (one pass), or null
-// (a second pass recomputes the picks' raw scores).
-template <int G>
-int launch_fast(const RouteArgs& a, hipStream_t s) {
-  const size_t smem = FastLayout::total(a.K);
-  auto kern = route_topk_fast_kernel<G>;
+template <int NT, int QT>
+int launch_heads(const RouteArgs& a, hipStream_t s) {
+  using Lay = HeadsLayout<NT, QT>;
+  const size_t smem = Lay::total(a.G, a.K);
+  auto kern = route_heads_kernel<NT, QT>;
   if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess)
     return MRSA_ERR_LAUNCH;
-  dim3 grid((unsigned)((a.L + kFastQ - 1) / kFastQ), (unsigned)a.Hkv, (unsigned)a.B);
-  hipLaunchKernelGGL(kern, grid, dim3(kFastThreads), smem, s, a);
+  dim3 grid((unsigned)((a.L + Lay::kQ - 1) / Lay::kQ), (unsigned)a.Hkv, (unsigned)a.B);
+  hipLaunchKernelGGL(kern, grid, dim3(kHeadThreads), smem, s, a, Lay::bias(a.G),
+                     Lay::picks(a.G));
   return mrsa_launch_status();
+}
+
+template <int G>
+int launch_tile(const RouteArgs& a, hipStream_t s) {
+  const size_t smem = TileLayout::total(a.K);
+  auto kern = route_tile_kernel<G>;
+  if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
+                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess)
+    return MRSA_ERR_LAUNCH;
+  dim3 grid((unsigned)((a.L + kTileQ - 1) / kTileQ), (unsigned)a.Hkv, (unsigned)a.B);
+  hipLaunchKernelGGL(kern, grid, dim3(kTileThreads), smem, s, a);
+  return mrsa_launch_status();
+}
+
+// The one-pass kernels.  At 7 heads x 4 KV heads, K = 32 (us, route_tile /
+// route_heads): 1024 queries x 16 chunks 55 / 9, 8064 x 63 77 / 39, 8192 x 128
+// 77 / 53, 32 x 128 66 / 13; 8192 x 256 79 / 98, 16384 x 256 157 / 198.  A
+// wave of route_tile keeps all 256 chunks of its 16 queries for every head, so
+// it pays for 256 chunks whatever C is and needs 256 workgroups of 128 queries
+// to fill the chip; route_heads pays per chunk and forms each logit once, but
+// reads the landmarks once per 16 or 32 queries.
+constexpr int64_t kTileMinGroups = 256;
+// 32 queries per workgroup of route_heads where that fills the chip twice.
+constexpr int64_t kHeadsWide = 512;
+
+int launch_fast(const RouteArgs& a, hipStream_t s) {
+  const bool wide = (a.L + 31) / 32 * a.Hkv * a.B >= kHeadsWide;
+  if (a.C <= 64) return wide ? launch_heads<4, 2>(a, s) : launch_heads<4, 1>(a, s);
+  if (a.C <= 128) return wide ? launch_heads<8, 2>(a, s) : launch_heads<8, 1>(a, s);
+  if (a.G >= 7 && (a.L + kTileQ - 1) / kTileQ * a.Hkv * a.B >= kTileMinGroups)
+    return a.G == 7 ? launch_tile<7>(a, s) : launch_tile<8>(a, s);
+  return launch_heads<16, 1>(a, s);
+}
+
+// Rows (token, KV head, batch) from which the scan path (128 queries per
+// workgroup) replaces the logits + workgroup selection, which spreads few rows
+// over more of the chip.
+constexpr int64_t kScanRows = 4096;
+
+template <int G>
+int launch_scan(const RouteArgs& a, float* ws, hipStream_t s) {
+  const int Cp = (int)scan_chunks(a.C);
+  const unsigned blocks = (unsigned)((a.L + kScanQ - 1) / kScanQ);
+  float* best = ws;                                  // [B, L, Hkv, Cp]
+  float* total = ws + a.B * a.L * a.Hkv * (int64_t)Cp;  // [B, L, Hkv, G]
+  int st;
+  if (!a.pre_softmax) {
+    hipLaunchKernelGGL(route_lse_kernel, dim3(blocks, (unsigned)(a.Hkv * G), (unsigned)a.B),
+                       dim3(kScanThreads), 0, s, a, total);
+    st = mrsa_launch_status();
+    if (st != MRSA_OK) return st;
+  }
+  const size_t smem = ScanLayout<G>::kTotal;
+  auto scan = route_scan_kernel<G>;
+  if (hipFuncSetAttribute(reinterpret_cast<const void*>(scan),
+                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess)
+    return MRSA_ERR_LAUNCH;
+  hipLaunchKernelGGL(scan, dim3(blocks, (unsigned)a.Hkv, (unsigned)a.B), dim3(kScanThreads), smem,
+                     s, a, a.pre_softmax ? nullptr : total, best, Cp);
+  st = mrsa_launch_status();
+  if (st != MRSA_OK) return st;
+  dim3 g2((unsigned)((a.L + 3) / 4), (unsigned)a.Hkv, (unsigned)a.B);
+  auto pick = a.C <= 256    ? route_pick_kernel<G, 4>
+              : a.C <= 1024 ? route_pick_kernel<G, 16>
+              : a.C <= 2048 ? route_pick_kernel<G, 32>
+                            : route_pick_kernel<G, 64>;
+  hipLaunchKernelGGL(pick, g2, dim3(256), 0, s, a, best, Cp);
+  return mrsa_launch_status();
+}
+
+int launch_scan(const RouteArgs& a, float* best, hipStream_t s) {
+  switch (a.G) {
+    case 1: return launch_scan<1>(a, best, s);
+    case 2: return launch_scan<2>(a, best, s);
+    case 3: return launch_scan<3>(a, best, s);
+    case 4: return launch_scan<4>(a, best, s);
+    case 5: return launch_scan<5>(a, best, s);
+    case 6: return launch_scan<6>(a, best, s);
+    case 7: return launch_scan<7>(a, best, s);
+    default: return launch_scan<8>(a, best, s);
+  }
 }
 
 }  // namespace
@@ -1480,9 +2165,21 @@ bool fast_path(const void* q, const void* lmk, int64_t chunks, int64_t kv_heads,
                int64_t head_dim, int64_t topk, int is_causal, int scores_fp32) {
   const bool aligned = ((uintptr_t)q % 16 == 0) && ((uintptr_t)lmk % 16 == 0);
   // (a batch's landmark keys, read through one buffer resource, stay under 2 GB)
-  return !scores_fp32 && !is_causal && head_dim == 128 && chunks <= 256 &&
-         topk <= kFastMaxTopk && aligned && (groups == 7 || groups == 8) &&
+  return !scores_fp32 && !is_causal && head_dim == 128 && chunks <= kFastMaxChunks &&
+         topk <= kFastMaxTopk && aligned && groups <= 8 &&
          chunks * kv_heads * groups * head_dim * 2 < ((int64_t)1 << 31);
+}
+
+// Shapes the scan path serves (it needs a workspace of scan_bytes).
+bool scan_path(int64_t batch, int64_t seq_len, int64_t chunks, int64_t kv_heads, int64_t groups,
+               int64_t head_dim, int64_t topk) {
+  return head_dim == 128 && groups <= 8 && topk <= kFastMaxTopk && chunks <= kScanMaxChunks &&
+         batch * seq_len * kv_heads >= kScanRows && kv_heads * groups <= 65535 &&
+         chunks * kv_heads * groups * head_dim * 2 < ((int64_t)1 << 31);
+}
+int64_t scan_bytes(int64_t batch, int64_t seq_len, int64_t chunks, int64_t kv_heads,
+                   int64_t groups) {
+  return batch * seq_len * kv_heads * (scan_chunks(chunks) + groups) * 4;
 }
 
 int route_topk_dispatch(const void* q, const void* lmk, const float* lse_local, const float* bias,
@@ -1527,11 +2224,18 @@ int route_topk_dispatch(const void* q, const void* lmk, const float* lse_local, 
   a.indices = indices;
   a.scores = scores;
   a.scores_fp32 = scores_fp32;
-  a.vec_out = topk % 32 == 0 && (uintptr_t)indices % 16 == 0 && (uintptr_t)scores % 16 == 0;
+  a.vec32_out =
+      topk % 32 == 0 && (uintptr_t)indices % 16 == 0 && (uintptr_t)scores % 16 == 0;
+  a.vec_out = topk % 8 == 0 && (uintptr_t)scores % 16 == 0;
   hipStream_t s = (hipStream_t)stream;
 
   const bool aligned = ((uintptr_t)q % 16 == 0) && ((uintptr_t)lmk % 16 == 0);
-  if (fast_path(q, lmk, chunks, kv_heads, groups, head_dim, topk, is_causal, scores_fp32)) return groups == 7 ? launch_fast<7>(a, s) : launch_fast<8>(a, s);
+  if (fast_path(q, lmk, chunks, kv_heads, groups, head_dim, topk, is_causal, scores_fp32)) 
+    return launch_fast(a, s);
+  if (workspace && (uintptr_t)workspace % 16 == 0 && aligned && seq_len <= 0x7fffffff &&
+      scan_path(batch, seq_len, chunks, kv_heads, groups, head_dim, topk) &&
+      workspace_bytes >= scan_bytes(batch, seq_len, chunks, kv_heads, groups))
+    return launch_scan(a, (float*)workspace, s);
   const bool block = workspace && head_dim == 128 && groups <= 8 && aligned &&
                      chunks <= (int64_t)kSelThreads * kSelMaxPer && seq_len <= 0x7fffffff &&
                      (uintptr_t)workspace % 16 == 0 &&
@@ -1569,6 +2273,20 @@ extern "C" int mrsa_route_topk_fwd(const void* q, const void* lmk, const float* 
 extern "C" int64_t mrsa_route_topk_workspace_bytes(int64_t batch, int64_t seq_len, int64_t chunks,
                                                    int64_t kv_heads, int64_t groups) {
   if (batch < 0 || seq_len < 0 || chunks < 0 || kv_heads < 0 || groups < 0) return -1;
+  return batch * seq_len * kv_heads * groups * chunks * 4;
+}
+
+extern "C" int64_t mrsa_route_topk_needed_bytes(int64_t batch, int64_t seq_len, int64_t chunks,
+                                                int64_t kv_heads, int64_t groups,
+                                                int64_t head_dim, int64_t topk, int is_causal,
+                                                int scores_fp32) {
+  if (batch < 0 || seq_len < 0 || chunks < 0 || kv_heads < 0 || groups < 0) return -1;
+  if (!scores_fp32 && !is_causal && head_dim == 128 && chunks <= kFastMaxChunks &&
+      topk <= kFastMaxTopk && groups <= 8)
+    return 0;
+  if (scan_path(batch, seq_len, chunks, kv_heads, groups, head_dim, topk))
+    return scan_bytes(batch, seq_len, chunks, kv_heads, groups);
+  if (head_dim != 128 || groups > 8 || chunks > (int64_t)kSelThreads * kSelMaxPer) return 0;
   return batch * seq_len * kv_heads * groups * chunks * 4;
 }
 
@@ -1620,8 +2338,8 @@ extern "C" int mrsa_route_topk_noalloc_fwd(
   // logits [batch, seq_len, kv_heads, groups, chunks] of the short-block path.
   // The one-pass matrix-core path runs without one (the dispatcher's own
   // test decides).  A problem that needs more than the static buffer is
-  // rejected.
-  const int64_t need = fast_path(q, lmk, chunks, kv_heads, groups, head_dim, topk, is_causal, scores_fp32)
+  // rejected (by this rule also where the call would take less of it).
+  const int64_t need = groups >= 7 && fast_path(q, lmk, chunks, kv_heads, groups, head_dim, topk, is_causal, scores_fp32)
                            ? 0
                            : batch * seq_len * kv_heads * groups * chunks * 4;
   if (need > (int64_t)MRSA_ROUTE_TOPK_SCRATCH_BYTES) return MRSA_ERR_SCRATCH;

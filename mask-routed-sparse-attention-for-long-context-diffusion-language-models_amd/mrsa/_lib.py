@@ -58,6 +58,7 @@ SIGNATURES = {
          _I64, _I, _I, _I64, _I64, _I, _F, _P, _P, _I, _P],
     ),
     "mrsa_route_topk_workspace_bytes": (_I64, [_I64, _I64, _I64, _I64, _I64]),
+    "mrsa_route_topk_needed_bytes": (_I64, [_I64] * 7 + [_I, _I]),
     "mrsa_route_topk_ws_fwd": (
         _I,
         [_P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64,

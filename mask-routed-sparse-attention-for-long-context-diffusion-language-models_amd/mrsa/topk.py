@@ -19,28 +19,18 @@ import torch
 from . import _lib
 from .kernel_utils import group_pad_to
 
-# Largest fp32 logits workspace the workspace route path may take (a 64k-token
-# Dream layer with 1024 chunks needs 7.5 GB of the 288 GB of HBM; the scalar
-# general kernel it replaces is about 50x slower there).
+# Largest workspace the route path may take of the 288 GB of HBM (beyond it
+# the scalar general kernel runs).
 _WORKSPACE_LIMIT = 16 << 30
 
 
-def _fast_shape(C, G, D, topk, scores_fp32, is_causal):
-    """Shapes of the matrix-core route kernel (up to 256 chunks, bf16 scores)."""
-    return (not scores_fp32 and not is_causal and D == 128 and C <= 256 and topk <= 64
-            and G in (7, 8))
-
-
 def _workspace_bytes(B, L, C, Hkv, G, D, topk, scores_fp32, is_causal):
-    """Bytes of the workspace the route kernels take, 0 for none.  The
-    matrix-core kernel (up to 256 chunks) runs without one; beyond 256
-    chunks, with head_dim 128, groups <= 8 and chunks <= 4096, the two-kernel
-    path runs over an fp32 logits workspace [B, L, Hkv, G, C]."""
-    if _fast_shape(C, G, D, topk, scores_fp32, is_causal):
-        return 0
-    if D != 128 or G > 8 or C > 4096:
-        return 0
-    n = B * L * Hkv * G * C * 4
+    """Bytes of the workspace the route kernels take, 0 for none: the fp32
+    selection scores [B, L, Hkv, C] of many rows against more than 256 chunks
+    (1.07 GB for a 64k-token layer with 1024 chunks), the fp32 logits
+    [B, L, Hkv, G, C] of a short block."""
+    n = int(_lib.call("mrsa_route_topk_needed_bytes", B, L, C, Hkv, G, D, topk,
+                      1 if is_causal else 0, 1 if scores_fp32 else 0))
     return n if n <= _WORKSPACE_LIMIT else 0
 
 
@@ -71,9 +61,8 @@ def route_topk_launch(
     drop mask of remote_drop_mask(key_valid, derive_window, block_size) is
     computed inside the kernel instead.
     Returns indices [B, L, Hkv, topk] int32 and scores [B, L, Hkv, G, topk].
-    ``use_workspace`` (None: by shape) passes the kernels an fp32 logits
-    workspace [B, L, Hkv, G, C] for the short-block path; the matrix-core
-    kernel (up to 256 chunks) takes none.
+    ``use_workspace`` (None: by shape) passes the kernels a workspace; the
+    one-pass kernel (up to 256 chunks) takes none.
     """
 
     if selection_mode not in {"post_softmax", "pre_softmax"}:
@@ -208,9 +197,6 @@ def _route_topk_impl(q5, lmks, lse4, bias4, drop_mask, key_valid, topk, block_si
     if use_workspace is None:
         use_workspace = nbytes > 0
     if use_workspace:
-        if not _fast_shape(C, G, D, topk, scores_fp32, is_causal):
-            nbytes = _lib.call("mrsa_route_topk_workspace_bytes", B, L, C, Hkv, G)
-        nbytes = max(int(nbytes), 0)
         ws = torch.empty((nbytes + 3) // 4, dtype=torch.float32, device=q5.device)
         st = _lib.call("mrsa_route_topk_ws_fwd", *args, _lib.ptr(ws), nbytes,
                        _lib.stream_of(qc))

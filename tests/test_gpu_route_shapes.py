@@ -1,0 +1,52 @@
+"""Route scoring and top-k at the edges of its kernels' ranges (16-chunk tiles,
+64 / 128 / 256-chunk instances, 16 or 32 queries per workgroup, the scan path's
+16- and 64-chunk stages) against the CPU oracle."""
+
+import pytest
+import torch
+
+from oracle import mrsa_oracle as O
+
+pytestmark = pytest.mark.gpu
+
+if torch.cuda.is_available():
+    from mrsa.topk import route_topk_launch
+
+DEV = "cuda:0"
+NEAR_TIE = 1e-5
+
+
+@pytest.mark.parametrize("B,L,C,Hkv,G,topk", [
+    (1, 1, 1, 1, 7, 8),            # one row, one chunk: slots past the picks are -1
+    (1, 17, 16, 2, 8, 16),
+    (2, 33, 64, 4, 7, 32),
+    (1, 4100, 64, 4, 4, 32),       # 32 queries per workgroup, last one partial
+    (1, 4097, 65, 4, 7, 32),
+    (1, 31, 128, 1, 1, 64),
+    (1, 130, 129, 3, 7, 20),       # a topk with no 16-byte output rows
+    (1, 50, 255, 2, 5, 32),
+    (1, 1025, 257, 4, 7, 32),      # scan path: C = 1 mod 16 and 64
+    (2, 683, 304, 3, 3, 24),
+    (1, 4099, 320, 1, 8, 64),
+])
+def test_route_topk_tile_edges_vs_oracle(B, L, C, Hkv, G, topk):
+    print(f"[gpu-case] route tile edges B={B} L={L} C={C} Hkv={Hkv} G={G} K={topk}", flush=True)
+    g = torch.Generator().manual_seed(1000 + L + C)
+    q5 = torch.randn(B, L, Hkv, G, 128, generator=g).bfloat16()
+    lmk = (0.5 * torch.randn(B, C, Hkv * G, 128, generator=g)).bfloat16()
+    lse4 = torch.randn(B, L, Hkv, G, generator=g) + 3.0
+    bias4 = torch.randn(B, C, Hkv, G, generator=g)
+    drop = (torch.rand(B, L, C, generator=g) < 0.2).to(torch.int32)
+    drop[:, L // 2] = 1  # a row with nothing to pick
+    idx, sc = route_topk_launch(q5.to(DEV), lmk.to(DEV), lse4.to(DEV), topk, 64,
+                                bias4=bias4.to(DEV), drop_mask=drop.to(DEV))
+    ridx, rsc, sel = O.route_topk(q5, lmk, lse4, topk, 64, drop_mask=drop, bias4=bias4)
+    idx = idx.cpu().long()
+    assert bool((idx[:, L // 2] == -1).all())
+    bad = (idx != ridx).any(-1)
+    assert int((bad & ~(O.boundary_gap(sel, topk) < NEAR_TIE)).sum()) == 0
+    ok = (~bad)[..., None, None].expand_as(rsc)
+    # bf16 scores of fp32 sums over 128 products: half a bf16 step (2^-9) plus
+    # the sums' own difference (below 1e-3 at these magnitudes)
+    torch.testing.assert_close(sc.cpu().float()[ok], rsc.bfloat16().float()[ok], atol=2e-3,
+                               rtol=2.0 ** -8)
