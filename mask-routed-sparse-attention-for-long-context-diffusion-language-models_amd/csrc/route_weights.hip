@@ -327,155 +327,234 @@ namespace {
 // plain form adds gG q_j / T to d remote_j (q = softmax of the remote logits)
 // and -gG / T to d local_lse; the affine form adds gG to dgate.
 // Rows whose outputs are constant (every logit masked; affine form with no
-// routed chunk) get zero gradients.  Gradients of the selected bias entries
-// are added atomically into d_bias, and the gate gradients into d_gate[0..1]
-// once per wave; both are zeroed by the caller.
-template <int LPR>
-__global__ void __launch_bounds__(256)
+// routed chunk) get zero gradients.
+//
+// A workgroup takes a range of tokens of one KV head.  The gradients of the
+// selected bias entries add up in an LDS copy of the head's [C][G] bias (LDS:
+// both fit kBwdLdsBytes, 960 chunks at G = 8) and reach d_bias with one atomic
+// per entry and workgroup, the gate gradients with one per workgroup; both are
+// zeroed by the caller.  One atomic per slot and one pair per wave took 742 us
+// at 16384 tokens x 28 heads x 32 slots (14.7 M adds onto 7168 bias entries,
+// 57 k onto the two gate words) where 180 MB are read and written; now 97 us.
+constexpr int kBwdThreads = 512;
+constexpr int64_t kBwdGroups = 512;         // two workgroups per CU
+constexpr int64_t kBwdLdsBytes = 60 * 1024;
+
+template <int LPR, bool LDS, bool VEC>
+__global__ void __launch_bounds__(kBwdThreads)
     route_weights_bwd_kernel(const uint16_t* __restrict__ scores,
                              const int32_t* __restrict__ indices, const float* __restrict__ bias,
                              const float* __restrict__ lse, const uint16_t* __restrict__ g_rw,
                              const uint16_t* __restrict__ g_lw, const float* __restrict__ g_gl,
-                             int64_t rows, int64_t L, int64_t C, int Hkv, int G, int K,
-                             float inv_t, const float* __restrict__ goff,
-                             const float* __restrict__ gsc, const float* __restrict__ e1,
-                             const float* __restrict__ e2, float* __restrict__ d_scores,
-                             float* __restrict__ d_bias, float* __restrict__ d_lse,
-                             float* __restrict__ d_gate) {
+                             int64_t L, int blocks, int tokens, int C, int Hkv, int G, int K, float inv_t,
+                             const float* __restrict__ goff, const float* __restrict__ gsc,
+                             const float* __restrict__ e1, const float* __restrict__ e2,
+                             float* __restrict__ d_scores, float* __restrict__ d_bias,
+                             float* __restrict__ d_lse, float* __restrict__ d_gate) {
+  extern __shared__ float lds[];  // LDS: the group's bias [C][G], then its gradient
+  __shared__ float gate_s[2];
   const int has_off = goff != nullptr, affine = gsc != nullptr;
   const float off = has_off ? *goff : 0.f;
   const float gscale = affine ? *gsc : 1.f;
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int part = (int)(t % LPR);
-  const int64_t r0 = t / LPR;
-  const bool live = r0 < rows;
-  const int64_t r = live ? r0 : rows - 1;  // lanes past the end join the reductions
-  const int Hq = Hkv * G;
-  const int hq = (int)(r % Hq);
-  const int64_t bl = r / Hq;
-  const int64_t b = bl / L;
-  const int hk = hq / G, g = hq - hk * G;
-  const int k0 = part * 8;
-  const int32_t* ix = indices + (bl * Hkv + hk) * K + k0;
+  const int tid = threadIdx.x, part = tid % LPR, k0 = part * 8;
+  const int bh = blockIdx.x / blocks;
+  const int64_t b = bh / Hkv;
+  const int hk = bh - (int)b * Hkv;
+  const int64_t l0 = (int64_t)(blockIdx.x - bh * blocks) * tokens;
+  const int nrows = (int)min((int64_t)tokens, L - l0) * G;  // rows (token, head of the group)
+  const int n = C * G;
+  const int64_t bias0 = (b * C * Hkv + hk) * G;             // of chunk 0; chunk stride Hkv G
+  const int64_t bstride = (int64_t)Hkv * G;
+  if constexpr (LDS) {
+    for (int i = tid; i < n; i += kBwdThreads) {
+      lds[i] = bias[bias0 + (i / G) * bstride + i % G];
+      lds[n + i] = 0.f;
+    }
+    __syncthreads();
+  }
+  float dscale_sum = 0.f, doff_sum = 0.f;
+  const int kl = K - 1;
+  for (int i0 = 0; i0 < nrows; i0 += kBwdThreads / LPR) {
+    const bool live = i0 + tid / LPR < nrows;
+    const int lr = min(i0 + tid / LPR, nrows - 1);  // lanes past the end join the reductions
+    const int tok = lr / G, g = lr - tok * G;
+    const int64_t bl = b * L + l0 + tok;
+    const int64_t r = (bl * Hkv + hk) * G + g;
+    const int32_t* ix = indices + (bl * Hkv + hk) * K;
 
-  // Loads are unconditional (clamped slots and chunks) and issued together:
-  // loads inside per-slot branches were each waited for at the branch end.
-  int32_t iv[8];
-  float x[8], gr[8];
-  float rmax = neg_inf();
-  const int64_t kl = K - 1;
+    // Loads are unconditional (clamped slots and chunks) and issued together:
+    // loads inside per-slot branches were each waited for at the branch end.
+    int32_t iv[8];
+    float x[8], gr[8];
+    float rmax = neg_inf();
+    float sc[8], bv[8], ex1[8], ex2[8];
+    if constexpr (VEC) {
+      // K % 8 == 0 and 16-byte aligned tensors: whole groups of 8 slots (lanes
+      // past the last read it again)
+      const int kk = min(k0, K - 8);
+      const u32x4_t i0v = *reinterpret_cast<const u32x4_t*>(ix + kk);
+      const u32x4_t i1v = *reinterpret_cast<const u32x4_t*>(ix + kk + 4);
+      const u32x4_t sv = *reinterpret_cast<const u32x4_t*>(scores + r * K + kk);
+      const u32x4_t gv = *reinterpret_cast<const u32x4_t*>(g_rw + r * K + kk);
 #pragma unroll
-  for (int j = 0; j < 8; ++j) iv[j] = ix[min((int64_t)j, kl - k0)];
-  float sc[8], bv[8], ex1[8], ex2[8];
+      for (int j = 0; j < 4; ++j) {
+        iv[j] = (int32_t)i0v[j];
+        iv[4 + j] = (int32_t)i1v[j];
+        sc[2 * j] = bf16_lo(sv[j]);
+        sc[2 * j + 1] = bf16_hi(sv[j]);
+        gr[2 * j] = bf16_lo(gv[j]);
+        gr[2 * j + 1] = bf16_hi(gv[j]);
+      }
+    } else {
 #pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    const int64_t kk = r * K + min((int64_t)(k0 + j), kl);
-    const bool ok = iv[j] >= 0 && iv[j] < C;
-    gr[j] = bf16_to_f32(g_rw[kk]);
-    sc[j] = bf16_to_f32(scores[kk]);
-    bv[j] = bias[((b * C + (ok ? iv[j] : 0)) * Hkv + hk) * G + g];
-    ex1[j] = e1 ? e1[kk] : 0.f;
-    ex2[j] = e2 ? e2[kk] : 0.f;
-  }
+      for (int j = 0; j < 8; ++j) {
+        const int kk = min(k0 + j, kl);
+        iv[j] = ix[kk];
+        sc[j] = bf16_to_f32(scores[r * K + kk]);
+        gr[j] = bf16_to_f32(g_rw[r * K + kk]);
+      }
+    }
 #pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    const bool in = k0 + j < K;
-    if (!in) iv[j] = -1;
-    if (!in) gr[j] = 0.f;
-    float y = sc[j] + bv[j];
-    if (e1) y += ex1[j];
-    if (e2) y += ex2[j];
-    const float v = in && iv[j] >= 0 && iv[j] < C ? y * inv_t : neg_inf();
-    x[j] = v;
-    rmax = fmaxf(rmax, v);
-  }
+    for (int j = 0; j < 8; ++j) {
+      const int kk = min(k0 + j, kl);
+      const int c = iv[j] >= 0 && iv[j] < C ? iv[j] : 0;
+      bv[j] = LDS ? lds[c * G + g] : bias[bias0 + c * bstride + g];
+      ex1[j] = e1 ? e1[r * K + kk] : 0.f;
+      ex2[j] = e2 ? e2[r * K + kk] : 0.f;
+    }
 #pragma unroll
-  for (int o = 1; o < LPR; o <<= 1) rmax = fmaxf(rmax, __shfl_xor(rmax, o, 64));
-  float local = lse[r];
-  if (has_off && !affine) local -= off;
-  local *= inv_t;
-  const float gl = g_lw ? bf16_to_f32(g_lw[r]) : 0.f;
-  const float gG = g_gl ? g_gl[r] : 0.f;
+    for (int j = 0; j < 8; ++j) {
+      const bool in = k0 + j < K;
+      if (!in) iv[j] = -1;
+      if (!in) gr[j] = 0.f;
+      float y = sc[j] + bv[j];
+      if (e1) y += ex1[j];
+      if (e2) y += ex2[j];
+      const float v = in && iv[j] >= 0 && iv[j] < C ? y * inv_t : neg_inf();
+      x[j] = v;
+      rmax = fmaxf(rmax, v);
+    }
+#pragma unroll
+    for (int o = 1; o < LPR; o <<= 1) rmax = fmaxf(rmax, __shfl_xor(rmax, o, 64));
+    float local = lse[r];
+    if (has_off && !affine) local -= off;
+    local *= inv_t;
+    const float gl = g_lw ? bf16_to_f32(g_lw[r]) : 0.f;
+    const float gG = g_gl ? g_gl[r] : 0.f;
 
-  // Branches are row-uniform, so the lane reductions inside stay within
-  // active lanes.
-  float dloc = 0.f, dscale = 0.f, doff = 0.f;
-  const float m = fmaxf(rmax, local);
-  if (m == neg_inf() || (affine && rmax == neg_inf())) {
+    // Branches are row-uniform, so the lane reductions inside stay within
+    // active lanes.
+    float dloc = 0.f, dscale = 0.f, doff = 0.f;
+    const float m = fmaxf(rmax, local);
+    if (m == neg_inf() || (affine && rmax == neg_inf())) {
 #pragma unroll
-    for (int j = 0; j < 8; ++j) x[j] = 0.f;
-  } else if (!affine) {
-    float sum = 0.f;
+      for (int j = 0; j < 8; ++j) x[j] = 0.f;
+    } else if (!affine) {
+      float sum = 0.f;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      x[j] = x[j] == neg_inf() ? 0.f : expf(x[j] - m);
-      sum += x[j];
+      for (int j = 0; j < 8; ++j) {
+        x[j] = x[j] == neg_inf() ? 0.f : expf(x[j] - m);
+        sum += x[j];
+      }
+#pragma unroll
+      for (int o = 1; o < LPR; o <<= 1) sum += __shfl_xor(sum, o, 64);
+      const float el = local == neg_inf() ? 0.f : expf(local - m);
+      sum += el;
+      float dot = 0.f;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        x[j] /= sum;
+        dot += x[j] * gr[j];
+      }
+#pragma unroll
+      for (int o = 1; o < LPR; o <<= 1) dot += __shfl_xor(dot, o, 64);
+      const float pl = el / sum;
+      dot += pl * gl;
+      // q_j = e_j / sum_remote e = x_j * sum / (sum - el); no remote chunk: 0.
+      const float rs = sum - el;
+      const float qf = rs > 0.f ? sum / rs : 0.f;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) x[j] = (x[j] * (gr[j] - dot) + gG * x[j] * qf) * inv_t;
+      dloc = (pl * (gl - dot) - gG) * inv_t;
+      doff = has_off ? -dloc : 0.f;
+    } else {
+      float sum = 0.f;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        x[j] = x[j] == neg_inf() ? 0.f : expf(x[j] - rmax);
+        sum += x[j];
+      }
+#pragma unroll
+      for (int o = 1; o < LPR; o <<= 1) sum += __shfl_xor(sum, o, 64);
+      const float rl = rmax + logf(sum);
+      const float gate = gscale * (rl - local) + (has_off ? off : 0.f);
+      const float mass = 1.f / (1.f + expf(-gate));
+      float qg = 0.f;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        x[j] /= sum;
+        qg += x[j] * gr[j];
+      }
+#pragma unroll
+      for (int o = 1; o < LPR; o <<= 1) qg += __shfl_xor(qg, o, 64);
+      const float dgate = (qg - gl) * mass * (1.f - mass) + gG;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) x[j] = x[j] * ((gr[j] - qg) * mass + dgate * gscale) * inv_t;
+      dloc = -dgate * gscale * inv_t;
+      dscale = dgate * (rl - local);
+      doff = has_off ? dgate : 0.f;
     }
+    if (live) {
+      float dx[8];
 #pragma unroll
-    for (int o = 1; o < LPR; o <<= 1) sum += __shfl_xor(sum, o, 64);
-    const float el = local == neg_inf() ? 0.f : expf(local - m);
-    sum += el;
-    float dot = 0.f;
+      for (int j = 0; j < 8; ++j) {
+        const bool valid = iv[j] >= 0 && iv[j] < C;
+        dx[j] = valid ? x[j] : 0.f;
+        if (valid && x[j] != 0.f) {
+          if constexpr (LDS)
+            __hip_atomic_fetch_add(lds + n + iv[j] * G + g, x[j], __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_WORKGROUP);
+          else
+            atomicAdd(&d_bias[bias0 + iv[j] * bstride + g], x[j]);
+        }
+      }
+      if constexpr (VEC) {
+        if (k0 < K) {
+          f32x4_t* dst = reinterpret_cast<f32x4_t*>(d_scores + r * K + k0);
+          dst[0] = f32x4_t{dx[0], dx[1], dx[2], dx[3]};
+          dst[1] = f32x4_t{dx[4], dx[5], dx[6], dx[7]};
+        }
+      } else {
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      x[j] /= sum;
-      dot += x[j] * gr[j];
+        for (int j = 0; j < 8; ++j)
+          if (k0 + j < K) d_scores[r * K + k0 + j] = dx[j];
+      }
+      if (part == 0) {
+        d_lse[r] = dloc;
+        dscale_sum += dscale;
+        doff_sum += doff;
+      }
     }
-#pragma unroll
-    for (int o = 1; o < LPR; o <<= 1) dot += __shfl_xor(dot, o, 64);
-    const float pl = el / sum;
-    dot += pl * gl;
-    // q_j = e_j / sum_remote e = x_j * sum / (sum - el); no remote chunk: 0.
-    const float rs = sum - el;
-    const float qf = rs > 0.f ? sum / rs : 0.f;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) x[j] = (x[j] * (gr[j] - dot) + gG * x[j] * qf) * inv_t;
-    dloc = (pl * (gl - dot) - gG) * inv_t;
-    doff = has_off ? -dloc : 0.f;
-  } else {
-    float sum = 0.f;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      x[j] = x[j] == neg_inf() ? 0.f : expf(x[j] - rmax);
-      sum += x[j];
-    }
-#pragma unroll
-    for (int o = 1; o < LPR; o <<= 1) sum += __shfl_xor(sum, o, 64);
-    const float rl = rmax + logf(sum);
-    const float gate = gscale * (rl - local) + (has_off ? off : 0.f);
-    const float mass = 1.f / (1.f + expf(-gate));
-    float qg = 0.f;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      x[j] /= sum;
-      qg += x[j] * gr[j];
-    }
-#pragma unroll
-    for (int o = 1; o < LPR; o <<= 1) qg += __shfl_xor(qg, o, 64);
-    const float dgate = (qg - gl) * mass * (1.f - mass) + gG;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) x[j] = x[j] * ((gr[j] - qg) * mass + dgate * gscale) * inv_t;
-    dloc = -dgate * gscale * inv_t;
-    dscale = dgate * (rl - local);
-    doff = has_off ? dgate : 0.f;
-  }
-  if (live) {
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      if (k0 + j >= K) continue;
-      const bool valid = iv[j] >= 0 && iv[j] < C;
-      d_scores[r * K + k0 + j] = valid ? x[j] : 0.f;
-      if (valid && x[j] != 0.f) atomicAdd(&d_bias[((b * C + iv[j]) * Hkv + hk) * G + g], x[j]);
-    }
-    if (part == 0) d_lse[r] = dloc;
   }
   if (d_gate) {
-    const bool mine = live && part == 0;
-    dscale = wave_sum(mine ? dscale : 0.f);
-    doff = wave_sum(mine ? doff : 0.f);
-    if ((threadIdx.x & 63) == 0) {
-      if (affine) atomicAdd(&d_gate[0], dscale);
-      if (has_off) atomicAdd(&d_gate[1], doff);
+    dscale_sum = wave_sum(dscale_sum);
+    doff_sum = wave_sum(doff_sum);
+    if (tid < 2) gate_s[tid] = 0.f;
+    __syncthreads();
+    if ((tid & 63) == 0) {
+      atomicAdd(&gate_s[0], dscale_sum);
+      atomicAdd(&gate_s[1], doff_sum);
+    }
+  }
+  __syncthreads();
+  if (d_gate && tid == 0) {
+    if (affine) atomicAdd(&d_gate[0], gate_s[0]);
+    if (has_off) atomicAdd(&d_gate[1], gate_s[1]);
+  }
+  if constexpr (LDS) {
+    for (int i = tid; i < n; i += kBwdThreads) {
+      const float v = lds[n + i];
+      if (v != 0.f) atomicAdd(&d_bias[bias0 + (i / G) * bstride + i % G], v);
     }
   }
 }
@@ -502,16 +581,29 @@ int route_weights_bwd(const void* scores, const int32_t* indices, const float* p
     return MRSA_ERR_INVALID_ARGUMENT;
   hipStream_t s = (hipStream_t)stream;
   const int lanes = (int)((topk + 7) / 8);
+  // About kBwdGroups workgroups in all, each with at least as many tokens as
+  // keep its threads busy once.
+  const int64_t split = std::max<int64_t>(1, kBwdGroups / (kv_heads * batch));
+  const int64_t tokens = std::max<int64_t>((seq_len + split - 1) / split, 16);
+  const int64_t blocks = (seq_len + tokens - 1) / tokens;
+  if (blocks * kv_heads * batch > 0x7fffffff || tokens * groups > 0x7fffffff)
+    return MRSA_ERR_UNSUPPORTED;
+  const dim3 grid((unsigned)(blocks * kv_heads * batch));
+  const bool lds = 8 * chunks * groups <= kBwdLdsBytes;
+  const bool vec = topk % 8 == 0 && ((uintptr_t)scores | (uintptr_t)indices |
+                                     (uintptr_t)grad_remote | (uintptr_t)d_scores) % 16 == 0;
   auto go = [&](auto lpr) {
     constexpr int LPR = decltype(lpr)::value;
-    const int64_t blocks = (rows * LPR + 255) / 256;
-    if (blocks > 0x7fffffff) return (int)MRSA_ERR_UNSUPPORTED;
-    hipLaunchKernelGGL(route_weights_bwd_kernel<LPR>, dim3((unsigned)blocks), dim3(256), 0, s,
+    auto kern = lds ? (vec ? route_weights_bwd_kernel<LPR, true, true>
+                           : route_weights_bwd_kernel<LPR, true, false>)
+                    : (vec ? route_weights_bwd_kernel<LPR, false, true>
+                           : route_weights_bwd_kernel<LPR, false, false>);
+    hipLaunchKernelGGL(kern, grid, dim3(kBwdThreads), lds ? (size_t)(8 * chunks * groups) : 0, s,
                        (const uint16_t*)scores, indices, prior_bias, local_lse,
                        (const uint16_t*)grad_remote, (const uint16_t*)grad_local,
-                       grad_gate_logit, rows, seq_len, chunks, (int)kv_heads, (int)groups,
-                       (int)topk, 1.f / temperature, gate_offset, gate_scale, value_bonus,
-                       selected_gumbel, d_scores, d_bias, d_local_lse,
+                       grad_gate_logit, seq_len, (int)blocks, (int)tokens, (int)chunks, (int)kv_heads,
+                       (int)groups, (int)topk, 1.f / temperature, gate_offset, gate_scale,
+                       value_bonus, selected_gumbel, d_scores, d_bias, d_local_lse,
                        (gate_scale || gate_offset) ? d_gate : nullptr);
     return mrsa_launch_status();
   };
