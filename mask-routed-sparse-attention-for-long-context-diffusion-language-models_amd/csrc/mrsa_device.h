@@ -73,8 +73,10 @@ __device__ __forceinline__ f32x4_t zero4() {
 // lane of the wave must be active.
 template <int CTRL>
 __device__ __forceinline__ float dpp_mov(float v) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CTRL, 0xf,
-                                                            0xf, false));
+  // (bound_ctrl with every row and bank on: the compiler folds the move into
+  // the add or max that uses it)
+  return __builtin_bit_cast(
+      float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
 }
 __device__ __forceinline__ float group16_max(float v) {
   v = fmaxf(v, dpp_mov<0xb1>(v));   // quad_perm [1,0,3,2]
@@ -101,7 +103,7 @@ __device__ __forceinline__ int group16_sum_i(int v) {
 // half-row.  Every lane of the wave must be active.
 template <int CTRL>
 __device__ __forceinline__ int dpp_mov_i(int v) {
-  return __builtin_amdgcn_mov_dpp(v, CTRL, 0xf, 0xf, false);
+  return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xf, 0xf, true);
 }
 __device__ __forceinline__ int group8_sum_i(int v) {
   v += dpp_mov_i<0xb1>(v);   // quad_perm [1,0,3,2]

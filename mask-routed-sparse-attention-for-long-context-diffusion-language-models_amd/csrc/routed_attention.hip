@@ -120,8 +120,8 @@ struct RaArgs {
   int det;                   // fixed accumulation order (per-query tickets instead of the lock)
   const float* slope;        // [Hq] ALiBi slopes (ALIBI instances only)
   // EXT instances (the routed backward's dQ walk): P^T tiles read from
-  // ext_p [B, Lq, Hq, K] records of 64 bf16 (lane group g's 16 keys at 16 g,
-  // in the order tile_P packs them), the fragments' V half being K^T, and
+  // ext_p [B, Lq, Hq, K] records of 64 bf16 (key 32 t + 16 m + j at
+  // 32 t + 2 j + m), the fragments' V half being K^T, and
   // the fp32 rows added into ext_out [B, Lq, Hq, 128].
   const uint16_t* ext_p;
   float* ext_out;
@@ -780,13 +780,13 @@ __global__ void __launch_bounds__(kThreads, 1) routed_attn_kernel(RaArgs a) {
     const int qq = it_q[ii];
     return a.ext_p +
            ((b * a.Lq + q0 + qq) * a.Hq + (int64_t)h * G + (gcol < G ? gcol : 0)) * K * 64 +
-           16 * grp;
+           8 * grp;
   };
   // the record of item ii's column (issued a tile ahead of its use)
   auto ext_load = [&](int ii, u32x4_t (&Pb)[2]) {
     const uint16_t* rec = ext_rec(ii) + it_slot[ii] * 64;
     Pb[0] = *reinterpret_cast<const u32x4_t*>(rec);
-    Pb[1] = *reinterpret_cast<const u32x4_t*>(rec + 8);
+    Pb[1] = *reinterpret_cast<const u32x4_t*>(rec + 32);
   };
   // padding columns zeroed; the later duplicate slots' records added
   auto ext_finish = [&](int ii, bool cvalid, u32x4_t (&Pb)[2]) {
@@ -808,7 +808,7 @@ __global__ void __launch_bounds__(kThreads, 1) routed_attn_kernel(RaArgs a) {
         const int s2 = __builtin_ctzll(dm);
         dm &= dm - 1ull;
         const u32x4_t y0 = *reinterpret_cast<const u32x4_t*>(rec0 + s2 * 64);
-        const u32x4_t y1 = *reinterpret_cast<const u32x4_t*>(rec0 + s2 * 64 + 8);
+        const u32x4_t y1 = *reinterpret_cast<const u32x4_t*>(rec0 + s2 * 64 + 32);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           f[0][2 * i] += bf16_lo(y0[i]);
@@ -821,6 +821,17 @@ __global__ void __launch_bounds__(kThreads, 1) routed_attn_kernel(RaArgs a) {
       for (int h2 = 0; h2 < 2; ++h2)
 #pragma unroll
         for (int i = 0; i < 4; ++i) Pb[h2][i] = pack_bf16x2(f[h2][2 * i], f[h2][2 * i + 1]);
+    }
+    // Record order -> operand order: word jj of half t holds keys 32 t + 4 grp
+    // + jj (low) and 16 more (high), the operand's elements jj and 4 + jj of
+    // k-step t.
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const u32x4_t d = Pb[t];
+      Pb[t][0] = __builtin_amdgcn_perm(d[1], d[0], 0x05040100u);
+      Pb[t][1] = __builtin_amdgcn_perm(d[3], d[2], 0x05040100u);
+      Pb[t][2] = __builtin_amdgcn_perm(d[1], d[0], 0x07060302u);
+      Pb[t][3] = __builtin_amdgcn_perm(d[3], d[2], 0x07060302u);
     }
   };
 

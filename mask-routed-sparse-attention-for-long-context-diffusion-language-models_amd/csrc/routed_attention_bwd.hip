@@ -4,20 +4,19 @@
 // (the forward kernel's semantics: a list ends at its first negative entry,
 // entries >= kv_len / 64 are skipped, the landmark slot and invalid / dropped
 // keys are not visible).  The backward follows the reference kernel
-// ops/hils_fwd_bwd_head.py:573-910 and its rounding points:
-//   P      = 2^(s c - lse) over the visible keys (lse = log2-sum-exp of the
-//            chunk, recomputed here), rounded to bf16;
+// ops/hils_fwd_bwd_head.py:573-910, which also rounds P and w dO to bf16:
+//   P      = softmax over the visible keys (recomputed here, fp32);
 //   dP     = dO . V^T (fp32);  di = sum_s P dP  ->  dW[q, g, k] = di (bf16);
 //   dS     = bf16(scale * w * P * (dP - di));
 //   dQ    += dS . K            (fp32, summed over the query's chunks);
-//   dK    += dS^T . Q,  dV += P^T . bf16(w * dO)  (fp32, summed over the
+//   dK    += dS^T . Q,  dV += bf16(w * P)^T . dO  (fp32, summed over the
 //            (query, slot) pairs that route to the chunk).
 // A chunk listed twice is processed once per slot (its gradient terms add,
 // as the weights do in the forward).
 //
 // Work split (chunk-major).  A list of the (query, slot) pairs of every
 // chunk is built first (count, scan, fill); a workgroup then owns one chunk
-// (or a segment of kSegEntries of its pairs) and recomputes each pair's
+// (or a segment of its pairs) and recomputes each pair's
 // chunk softmax:
 //   dK / dV  stay in the workgroup's registers and are written once per
 //            chunk (added with atomics when the chunk's pairs span several
@@ -37,15 +36,13 @@
 #include "mrsa_device.h"
 
 #include <algorithm>
+#include <type_traits>
 
 using namespace mrsa;
 
 namespace {
 
-constexpr int kWaves = 4;
-constexpr int kThreads = 64 * kWaves;
 constexpr int kMaxTopk = 64;
-constexpr uint32_t kFragBytes = 32768;
 
 struct BwdArgs {
   const uint16_t* q;
@@ -70,10 +67,11 @@ struct BwdArgs {
   const int32_t* start;      // [B * Hkv * Ck + 1]
   const int32_t* ustart;     // [B * Hkv * Ck + 1]
   const float* slope;        // [Hq] ALiBi slopes or null
-  // dS records [B, Lq, Hq, K] x 64 bf16 (lane group g's 16 keys at 16 g, in
-  // the packed P^T order of the forward's tiles), one per listed slot, for
-  // the dQ walk.
+  // dS records [B, Lq, Hq, K] x 64 bf16 (key 32 t + 16 m + j at 32 t + 2 j + m),
+  // one per listed slot, for the dQ walk.
   uint16_t* ds_rec;
+  uint16_t* sink;            // 256 elements nothing reads
+  int seg;                   // pairs per work unit
 };
 
 
@@ -81,82 +79,24 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* base, ui
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)bytes,
                                            (int)0x00020000);
 }
-__device__ __forceinline__ u32x4_t bload(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
-  return __builtin_amdgcn_raw_buffer_load_b128(r, (int)voff, (int)soff, 0);
-}
-// First-half images (K or V, keys x dims): image 4 mt + ks at 1024 (4 mt + ks).
-__device__ __forceinline__ void load_rows(u32x4_t (&x)[4][4], __amdgpu_buffer_rsrc_t r,
-                                          uint32_t lo, uint32_t cb) {
-#pragma unroll
-  for (int mt = 0; mt < 4; ++mt)
-#pragma unroll
-    for (int ks = 0; ks < 4; ++ks) x[mt][ks] = bload(r, lo + 1024u * ks, cb + 4096u * mt);
-}
 // Bits of the nonzero bytes (bit j = byte j) of one 64-byte keep / key-valid
 // row: one byte per lane and a wave ballot (every lane must be active).
 __device__ __forceinline__ uint64_t nonzero_bits(const int8_t* row) {
   return __builtin_amdgcn_ballot_w64(row[threadIdx.x & 63] != 0);
 }
 
-// One column tile's chunk gradient, in place.  S^T / dP^T lane (grp, j):
-// keys 16 mt + 4 grp + r of column j; msh bit 16 mt + r set = key excluded.
-//   S  <- P  = bf16(2^(s c - lse)) over the visible keys (0 when none is)
-//   dP <- dS = bf16(sw P (dP - di)),  di = sum P dP per column (returned)
-// With ALiBi (alibi, wave-uniform) the exp2-domain logit is s c + sl
-// max(0, 62 - key), sl = -slope[head] c for this lane's column
-// (ops/hils_fwd_bwd_head.py:755-760, the backward's bias term).
-__device__ __forceinline__ float chunk_grad(f32x4_t (&S)[4], f32x4_t (&dP)[4], uint64_t msh,
-                                            float c2, float sw, bool alibi = false,
-                                            float sl = 0.f, int grp = 0) {
-  if (alibi) {
-#pragma unroll
-    for (int mt = 0; mt < 4; ++mt)
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        S[mt][r] = __builtin_fmaf(
-            S[mt][r], c2, sl * fmaxf(0.f, (float)(62 - 16 * mt - r) - 4.f * (float)grp));
-    c2 = 1.f;
-  }
-  float mx = neg_inf();
-#pragma unroll
-  for (int mt = 0; mt < 4; ++mt)
-#pragma unroll
-    for (int r = 0; r < 4; ++r)
-      if (!((msh >> (16 * mt + r)) & 1ull)) mx = fmaxf(mx, S[mt][r] * c2);
-  mx = across4_max(mx);
-  float sum = 0.f;
-  if (mx != neg_inf()) {
-#pragma unroll
-    for (int mt = 0; mt < 4; ++mt)
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        if (!((msh >> (16 * mt + r)) & 1ull)) sum += exp2_hw(S[mt][r] * c2 - mx);
-  }
-  sum = across4_sum(sum);
-  const float lse = mx == neg_inf() ? neg_inf() : mx + log2_hw(sum);
-  float di = 0.f;
-#pragma unroll
-  for (int mt = 0; mt < 4; ++mt)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const bool vis = !((msh >> (16 * mt + r)) & 1ull) && lse != neg_inf();
-      const float p = vis ? bf16_to_f32(f32_to_bf16(exp2_hw(S[mt][r] * c2 - lse))) : 0.f;
-      S[mt][r] = p;
-      di += p * dP[mt][r];
-    }
-  di = across4_sum(di);
-#pragma unroll
-  for (int mt = 0; mt < 4; ++mt)
-#pragma unroll
-    for (int r = 0; r < 4; ++r)
-      dP[mt][r] = bf16_to_f32(f32_to_bf16(sw * S[mt][r] * (dP[mt][r] - di)));
-  return di;
-}
-
 // ---- chunk-major dK / dV ---------------------------------------------------
 constexpr int kListBlock = 256;       // queries per list workgroup (one per thread)
 constexpr int kMaxListChunks = 8192;  // LDS counters of the list kernels (32 KB)
-constexpr int kSegEntries = 1024;     // (query, slot) pairs per dK / dV work unit
+
+// (query, slot) pairs per dK / dV work unit: about 4096 units (16 per CU), at
+// least 256 pairs (a unit's K, V and dK / dV traffic) and at most 1024.  At
+// 16384 queries the backward takes 3.51 ms with 512, 3.61 with 1024, 0.5 more with
+// 2048.
+int64_t segment_entries(int64_t pairs) {
+  const int64_t n = (pairs / 4096 + 63) / 64 * 64;
+  return n < 256 ? 256 : n > 1024 ? 1024 : n;
+}
 
 // The valid slots of one index row: up to the first negative entry, chunks
 // below Ck.
@@ -193,9 +133,10 @@ __global__ void __launch_bounds__(kListBlock) list_count_kernel(BwdArgs a, int32
 }
 
 // 2. Exclusive scans over the chunks (b, h, c): list starts and work-unit
-//    starts (ceil(count / kSegEntries) units per chunk).  One workgroup.
+//    starts (ceil(count / seg) units per chunk).  One workgroup.
 __global__ void __launch_bounds__(1024) list_scan_kernel(const int32_t* count, int64_t N,
-                                                         int32_t* start, int32_t* ustart) {
+                                                         int seg, int32_t* start,
+                                                         int32_t* ustart) {
   __shared__ int32_t s1[1024], s2[1024];
   const int tid = threadIdx.x;
   const int64_t per = (N + 1023) / 1024;
@@ -203,7 +144,7 @@ __global__ void __launch_bounds__(1024) list_scan_kernel(const int32_t* count, i
   int32_t t1 = 0, t2 = 0;
   for (int64_t i = lo; i < hi; ++i) {
     t1 += count[i];
-    t2 += (count[i] + kSegEntries - 1) / kSegEntries;
+    t2 += (count[i] + seg - 1) / seg;
   }
   s1[tid] = t1;
   s2[tid] = t2;
@@ -220,7 +161,7 @@ __global__ void __launch_bounds__(1024) list_scan_kernel(const int32_t* count, i
     start[i] = r1;
     ustart[i] = r2;
     r1 += count[i];
-    r2 += (count[i] + kSegEntries - 1) / kSegEntries;
+    r2 += (count[i] + seg - 1) / seg;
   }
   if (tid == 1023) {
     start[N] = s1[1023];
@@ -249,59 +190,62 @@ __global__ void __launch_bounds__(kListBlock) list_fill_kernel(BwdArgs a, const 
     });
 }
 
-// Kept-key bits (bit j = key j kept) of one 64-byte token-keep row, per lane.
-__device__ __forceinline__ uint64_t keep_row_bits(const int8_t* kr) {
-  uint64_t bits = 0ull;
-#pragma unroll
-  for (int v = 0; v < 4; ++v) {
-    const u32x4_t x = *reinterpret_cast<const u32x4_t*>(kr + 16 * v);
-#pragma unroll
-    for (int w = 0; w < 4; ++w)
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        bits |= ((x[w] >> (8 * i)) & 0xffu) ? 1ull << (16 * v + 4 * w + i) : 0ull;
-  }
-  return bits;
+typedef __attribute__((address_space(3))) void lds_void_t;
+typedef short s16x4_t __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) s16x4_t lds_s16x4_t;
+
+// Four 16-bit values of one column out of four LDS rows (gfx950's transposing
+// read): lanes 16 g + i of a group point at 8-byte pieces, piece i & 3 of row
+// i >> 2; lane i receives element i of the four rows.
+__device__ __forceinline__ u32x2_t read_transposed(uint32_t addr) {
+  return __builtin_bit_cast(u32x2_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                                         (lds_s16x4_t*)(uintptr_t)addr));
+}
+__device__ __forceinline__ uint32_t lds_addr(const void* p) {
+  return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) char*)(p);
 }
 
-// LDS of the chunk-major kernel (bytes): the chunk's V images (16 KB, lane
-// l's 16 bytes of image i at 1024 i + 16 l) and one round's tiles, bf16
-// [row][64 columns] with 128-byte rows whose 16-byte block b sits at
-// b ^ ((row >> 1) & 7): P^T and dS^T (64 key rows), Q^T and bf16(w dO)^T
-// (128 dim rows).
-constexpr uint32_t kKvV = 0;
-constexpr uint32_t kKvPt = 16384;
-constexpr uint32_t kKvDs = kKvPt + 8192;
-constexpr uint32_t kKvQt = kKvDs + 8192;
-constexpr uint32_t kKvWd = kKvQt + 16384;
-constexpr uint32_t kKvBytes = kKvWd + 16384;
-
-__device__ __forceinline__ uint32_t tile_off(uint32_t base, int row, int col) {
-  return base + row * 128 + ((((col >> 3) ^ ((row >> 1) & 7))) << 4) + (col & 7) * 2;
-}
-__device__ __forceinline__ u32x4_t tile_read(const unsigned char* sm, uint32_t base, int row,
-                                             int blk) {
-  return *reinterpret_cast<const u32x4_t*>(sm + base + row * 128 +
-                                           ((blk ^ ((row >> 1) & 7)) << 4));
-}
-__device__ __forceinline__ void tile_put(unsigned char* sm, uint32_t base, int row, int col,
-                                         uint32_t v16) {
-  *reinterpret_cast<uint16_t*>(sm + tile_off(base, row, col)) = (uint16_t)v16;
+__device__ __forceinline__ u32x4_t lds_read16(uint32_t addr) {
+  return *(const __attribute__((address_space(3))) u32x4_t*)(uintptr_t)addr;
 }
 
-// One workgroup per work unit: chunk (b, h, c) and a segment of its pairs.
-// A round takes 8 pairs, two per wave (16 columns: pair 8 j >> 3, head j & 7):
-//   phase 1 (per wave): S^T = K . Q^T (K images in registers), dP^T = V . dO^T
-//     (V images from LDS), the chunk gradient, and the columns of P^T, dS^T,
-//     Q^T, bf16(w dO)^T into the round's tiles;
-//   phase 2 (wave w: dims 32 w .. + 31): dK += dS^T . Q, dV += P^T . bf16(w dO)
-//     over the round's 64 columns (two k-steps).
-template <bool ALIBI>
-__global__ void __launch_bounds__(kThreads, 2) routed_attn_dkv_kernel(BwdArgs a) {
-  __shared__ __attribute__((aligned(16))) unsigned char sm[kKvBytes];
+// One workgroup per work unit: chunk (b, h, c) and a segment of its pairs.  8
+// waves: wave 2 w + s takes keys 32 s .. 32 s + 31 of the pairs of group w, 4 a
+// round, as 32 matrix rows (row 8 p + g: pair p, head g):
+//   S = Q . K^T and dP = dO . V^T: lane (grp, j) gets rows 16 ct + 4 grp + r of
+//     keys 16 mt + j of its half; the rows' sums of p = 2^x and p dP over the
+//     16 lanes, and over the two halves through LDS;
+//   dK += dS^T . Q and dV += bf16(w P)^T . dO: a lane's rows are consecutive
+//     elements of the products' reduction, so dS and w P are operands as they
+//     leave the softmax, and Q and dO rows are read from LDS transposed.
+// Q and dO rows arrive by DMA in whole 256-byte rows, a round ahead (row r's
+// 16-byte part p at unit p ^ (r & 15)); half of a wave's K stays in registers,
+// the rest and V in LDS, its dK and dV (32 keys x 128 dims, fp32) in 128 accumulators, summed
+// over the four groups through LDS once per unit.  Halving the keys and not
+// the pairs is what lets two waves share a SIMD; with 64 keys per wave the 256
+// accumulators left no registers and the kernel ran 5090 us.  Bound: the Q and
+// dO rows, read once per routed slot (7.5 GB at 16384 queries x 28 heads x 32
+// slots, 60% of it past L2) beside 1.9 GB of records written; products and
+// VALU instructions take 55% of the cycles, LDS 26%.  Measured there: 2270 us;
+// with eight pairs per workgroup and round, element-wise transposes through LDS
+// and no prefetch 3410 us.
+constexpr int kGroups = 4;                 // pair groups of a workgroup
+constexpr int kDkvThreads = 128 * kGroups;
+constexpr int kPairs = 4;                  // per group and round
+constexpr uint32_t kRowsBytes = 32 * 256;  // one round's Q or dO rows of a group
+constexpr uint32_t kDkvK = 16384;          // K images of key tiles 1 and 3 (8 KB)
+constexpr uint32_t kDkvExch = 24576;       // [2][2 kGroups][3][32] f32 row sums
+constexpr uint32_t kDkvRows = kDkvExch + 2 * 2 * kGroups * 384;  // [group][2][Q, dO] rows
+constexpr uint32_t kDkvLds = kDkvRows + kGroups * 4 * kRowsBytes;
+static_assert(kDkvRows % 256 == 0 && kGroups * 32768 <= kDkvLds, "row alignment; the final sums");
+
+template <bool ALIBI, bool KEEP>
+__global__ void __launch_bounds__(kDkvThreads, 2) routed_attn_dkv_kernel(BwdArgs a) {
+  extern __shared__ __align__(256) unsigned char sm[];
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int wave = tid >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int group = wave >> 1, half = wave & 1;
   const int j = lane & 15, grp = lane >> 4;
   const int64_t N = a.B * a.Hkv * a.Ck;
   const int64_t u = blockIdx.x;
@@ -314,10 +258,10 @@ __global__ void __launch_bounds__(kThreads, 2) routed_attn_dkv_kernel(BwdArgs a)
     else hi = mid;
   }
   const int64_t bhc = lo;
-  const int64_t cs = a.start[bhc], ce = a.start[bhc + 1];
-  const int64_t e0 = cs + (u - a.ustart[bhc]) * kSegEntries;
-  const int64_t e1 = min(ce, e0 + kSegEntries);
-  const bool whole = ce - cs <= kSegEntries;
+  const int cs = a.start[bhc], ce = a.start[bhc + 1];
+  const int e0 = cs + (int)(u - a.ustart[bhc]) * a.seg;
+  const int e1 = min(ce, e0 + a.seg);
+  const bool whole = ce - cs <= a.seg;
   const int64_t c = bhc % a.Ck;
   const int64_t bh = bhc / a.Ck;
   const int h = (int)(bh % a.Hkv);
@@ -328,170 +272,337 @@ __global__ void __launch_bounds__(kThreads, 2) routed_attn_dkv_kernel(BwdArgs a)
   if (a.key_valid)
     excl |= ~nonzero_bits(reinterpret_cast<const int8_t*>(a.key_valid + b * a.Lk + c * 64));
   const uint32_t l16 = 16u * lane;
-  const uint32_t cb = (uint32_t)c * kFragBytes;
-  u32x4_t kb[4][4];
-  load_rows(kb, make_rsrc(a.fwd + (b * a.Hkv + h) * a.Ck * 16384, (uint32_t)a.Ck * kFragBytes),
-            l16, cb);
+  const unsigned char* kimg = reinterpret_cast<const unsigned char*>(
+      a.fwd + ((b * a.Hkv + h) * a.Ck + c) * 16384);
+  u32x4_t kb[4];  // K images of the half's first key tile
+#pragma unroll
+  for (int ks = 0; ks < 4; ++ks)
+    kb[ks] = *reinterpret_cast<const u32x4_t*>(kimg + 1024 * (8 * half + ks) + l16);
+  {
+    // the other one's: image (half, ks) at 1024 (4 half + ks)
+    const int o = 16 * tid;
+    *reinterpret_cast<u32x4_t*>(sm + kDkvK + o) = *reinterpret_cast<const u32x4_t*>(
+        kimg + 4096 + (o & 4095) + 2 * (o & 4096));
+  }
   {
     // the V images: the first half of the chunk's bwd fragment (16 KB)
-    const unsigned char* vsrc =
-        reinterpret_cast<const unsigned char*>(a.bwd + (b * a.Hkv + h) * a.Ck * 16384) + cb;
+    const unsigned char* vsrc = reinterpret_cast<const unsigned char*>(
+        a.bwd + ((b * a.Hkv + h) * a.Ck + c) * 16384);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int o = 16 * (tid + kThreads * i);
-      *reinterpret_cast<u32x4_t*>(sm + kKvV + o) = *reinterpret_cast<const u32x4_t*>(vsrc + o);
+    for (int i = 0; i < 16384 / 16 / kDkvThreads; ++i) {
+      const int o = 16 * (tid + kDkvThreads * i);
+      *reinterpret_cast<u32x4_t*>(sm + o) = *reinterpret_cast<const u32x4_t*>(vsrc + o);
     }
   }
-  f32x4_t dk[4][2], dv[4][2];
-#pragma unroll
-  for (int mt = 0; mt < 4; ++mt)
-#pragma unroll
-    for (int dt = 0; dt < 2; ++dt) {
-      dk[mt][dt] = zero4();
-      dv[mt][dt] = zero4();
-    }
   const float c2 = a.scale_log2;
-  const int g = j & 7;
-  const int col = 16 * wave + j;
-  __syncthreads();  // V images staged
+  const int g4 = 4 * (grp & 1);  // this lane's rows: heads g4 + r of pair 2 ct + phalf
+  const int phalf = grp >> 1;
+  const float ninf = neg_inf();
+  // 0, or -inf where key 16 mt + j of half t is excluded
+  auto mask_of = [&](int t, int mt) {
+    return ((excl >> (32 * t + 16 * mt + j)) & 1ull) ? ninf : 0.f;
+  };
+  const float madd[2] = {mask_of(half, 0), mask_of(half, 1)};
+  float sl[4];                   // ALiBi: -slope c2 of this lane's heads
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+    sl[r] = ALIBI ? -a.slope[(int64_t)h * G + min(g4 + r, G - 1)] * c2 : 0.f;
+  auto alibi = [&](int t, int mt, int r, float x) {
+    return ALIBI ? __builtin_fmaf(sl[r], fmaxf(0.f, (float)(62 - 32 * t - 16 * mt - j)), x) : x;
+  };
+  // DMA lane offsets: instruction k (0..7) fills rows 4 k + grp of the round
+  // (pair k >> 1, head 4 (k & 1) + grp; heads past G - 1 repeat it).
+  uint32_t voff[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k)
+    voff[k] = 256u * (uint32_t)min(4 * (k & 1) + grp, G - 1) +
+              16u * (uint32_t)(j ^ ((4 * k + grp) & 15));
+  unsigned char* rows = sm + kDkvRows + group * 4 * kRowsBytes;  // [2][Q, dO]
+  const int64_t row0 = b * a.Lq * a.Hq + (int64_t)h * G;         // row of query 0, head 0
+  // the first pair of this group's round i; absent pairs repeat the last one
+  auto base_of = [&](int i) { return e0 + kGroups * kPairs * i + kPairs * group; };
+  auto entry = [&](int i) { return a.list[min(base_of(i) + (lane & 3), e1 - 1)]; };
+  // half 0 brings the group's Q rows, half 1 its dO rows
+  const uint16_t* src = half ? a.dout : a.q;
+  auto stage = [&](const int32_t (&ent)[kPairs], int buf) {
+#pragma unroll
+    for (int p = 0; p < kPairs; ++p) {
+      const __amdgpu_buffer_rsrc_t rs = make_rsrc(
+          src + (row0 + (int64_t)(ent[p] & 0xffffff) * a.Hq) * 128, (uint32_t)G * 256u);
+#pragma unroll
+      for (int kk = 0; kk < 2; ++kk) {
+        const int k = 2 * p + kk;
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(
+            rs, (lds_void_t*)(rows + (2 * buf + half) * kRowsBytes + 1024 * k), 16, voff[k & 3], 0,
+            0, 0);
+      }
+    }
+  };
+  auto split = [&](int32_t v, int32_t (&ent)[kPairs]) {
+#pragma unroll
+    for (int p = 0; p < kPairs; ++p) ent[p] = __builtin_amdgcn_readlane(v, p);
+  };
+  // The routing weights of this lane's rows (raw; padding heads repeat the last)
+  auto load_w = [&](const int32_t (&ent)[kPairs], uint32_t (&w)[2][4]) {
+#pragma unroll
+    for (int ct = 0; ct < 2; ++ct) {
+      const int32_t v = phalf ? ent[2 * ct + 1] : ent[2 * ct];
+      const uint16_t* wp =
+          a.w + (row0 + (int64_t)(v & 0xffffff) * a.Hq + g4) * K + ((v >> 24) & 63);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) w[ct][r] = wp[min(r, G - 1 - g4) * K];
+    }
+  };
+  const unsigned char* vown = sm + 8192 * half + l16;  // V images of this wave's keys
+  const unsigned char* kown = sm + kDkvK + 4096 * half + l16;
+  f32x4_t dk[2][8], dv[2][8];
+#pragma unroll
+  for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+    for (int nt = 0; nt < 8; ++nt) {
+      dk[mt][nt] = zero4();
+      dv[mt][nt] = zero4();
+    }
+  int32_t ent[kPairs], ent2[kPairs], entn[kPairs];
+  const int rounds = (e1 - e0 + kGroups * kPairs - 1) / (kGroups * kPairs);
+  // One pass over the unit's pairs; true when some row's sum left fp32's range
+  // (never with STAB: p is then stabilised by each half's maximum).
+  auto pass = [&](auto stab) {
+    constexpr bool STAB = decltype(stab)::value;
+    bool fine = true;
+    split(entry(0), ent);
+    stage(ent, 0);
+    asm volatile("" ::: "memory");
+    int32_t evn = entry(1);
+    for (int i = 0; i < rounds; ++i) {
+      const int base = base_of(i);
+      const int buf = i & 1;
+      // This wave's rows of the round have landed: the round's entries, loaded
+      // after them, have been read.  The barrier covers the other waves' rows
+      // (and, first, the V and K images), and their reads of the buffers written
+      // next.
+      split(evn, entn);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      uint32_t wraw[2][4];
+      load_w(ent, wraw);
+      asm volatile("" ::: "memory");
+      stage(entn, buf ^ 1);
+      asm volatile("" ::: "memory");
+      evn = entry(i + 2);
+      asm volatile("" ::: "memory");
 
-  for (int64_t r0 = e0; r0 < e1; r0 += 8) {
-    // The tile addresses derive from lane values redefined each round, so
-    // they are formed where used rather than held in registers across rounds.
-    int lj = j, lg = grp, lc = col;
-    asm volatile("" : "+v"(lj), "+v"(lg), "+v"(lc));
-    // ---- phase 1
-    const int64_t e = r0 + 2 * wave + (j >> 3);
-    const bool have = e < e1;
-    const bool cvalid = have && g < G;
-    int64_t q = 0;
-    int k = 0;
-    if (have) {
-      const int32_t v = a.list[e];
-      q = v & 0xffffff;
-      k = (v >> 24) & 63;
-    }
-    const int64_t row = (b * a.Lq + q) * a.Hq + (int64_t)h * G + g;
-    u32x4_t Qb[4], Db[4];
+      // Addresses of this lane's operand rows (row j + 16 ct, part 4 ks + grp:
+      // ks flips bits 6 and 7), and below of the transposed reads.  Formed anew
+      // each round from a redefined lane number: held across rounds they spill,
+      // and a reload waits for every load and store in flight.
+      uint32_t lj = lane;
+      asm volatile("" : "+v"(lj));
+      const uint32_t arow = lds_addr(rows) + (uint32_t)buf * 2u * kRowsBytes + 256u * (lj & 15u) +
+                            16u * (((lj >> 4) ^ (lj & 3u)) | (lj & 12u));
+      // S = Q . K^T and dP = dO . V^T of 16 rows
+      auto products = [&](int ct, f32x4_t (&S)[2], f32x4_t (&dP)[2]) {
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
-      const u32x4_t z = {0u, 0u, 0u, 0u};
-      Qb[ks] = z;
-      Db[ks] = z;
-      if (cvalid) {
-        Qb[ks] = *reinterpret_cast<const u32x4_t*>(a.q + row * 128 + 32 * ks + 8 * grp);
-        Db[ks] = *reinterpret_cast<const u32x4_t*>(a.dout + row * 128 + 32 * ks + 8 * grp);
-      }
-    }
-    const float wv = cvalid ? bf16_to_f32(a.w[row * K + k]) : 0.f;
-    uint64_t ex = excl;
-    if (a.keep && have) ex |= ~keep_row_bits(a.keep + (((b * a.Lq + q) * a.Hkv + h) * K + k) * 64);
-    const uint64_t msh = ex >> (4 * grp);
-    f32x4_t S[4], dP[4];
+        for (int mt = 0; mt < 2; ++mt) S[mt] = dP[mt] = zero4();
 #pragma unroll
-    for (int mt = 0; mt < 4; ++mt) {
-      S[mt] = zero4();
+        for (int ks = 0; ks < 4; ++ks) {
+          const uint32_t at = (arow ^ (64u * ks)) + 4096u * ct;
+          const u32x4_t A = lds_read16(at), D = lds_read16(at + kRowsBytes);
 #pragma unroll
-      for (int ks = 0; ks < 4; ++ks) S[mt] = mfma_bf16_16x16x32(kb[mt][ks], Qb[ks], S[mt]);
-    }
-#pragma unroll
-    for (int mt = 0; mt < 4; ++mt) {
-      dP[mt] = zero4();
-#pragma unroll
-      for (int ks = 0; ks < 4; ++ks) {
-        const u32x4_t vi =
-            *reinterpret_cast<const u32x4_t*>(sm + kKvV + 1024 * (4 * mt + ks) + l16);
-        dP[mt] = mfma_bf16_16x16x32(vi, Db[ks], dP[mt]);
-      }
-    }
-#pragma unroll
-    for (int ks = 0; ks < 4; ++ks)
-#pragma unroll
-      for (int e8 = 0; e8 < 8; ++e8) {
-        const int dim = 32 * ks + 8 * lg + e8;
-        const uint32_t qv = (Qb[ks][e8 >> 1] >> (16 * (e8 & 1))) & 0xffffu;
-        const float dov = bf16_to_f32((Db[ks][e8 >> 1] >> (16 * (e8 & 1))) & 0xffffu);
-        tile_put(sm, kKvQt, dim, lc, qv);
-        tile_put(sm, kKvWd, dim, lc, f32_to_bf16(wv * dov));
-      }
-    const float sl = ALIBI && cvalid ? -a.slope[(int64_t)h * G + g] * c2 : 0.f;
-    const float di = chunk_grad(S, dP, msh, c2, a.scale * wv, ALIBI, sl, lg);  // S <- P, dP <- dS
-    if (cvalid && grp == 0) a.dw[row * K + k] = (uint16_t)f32_to_bf16(di);
-    // dS of this lane's column packed in the tiled key order (reduction
-    // index 8 grp + e of k-step ks is key 32 ks + 16 (e >> 2) + 4 grp +
-    // (e & 3)), the P^T operand order of the forward's tiles: stored as the
-    // column's record for the dQ walk.
-    {
-      u32x4_t Sb[2];
-#pragma unroll
-      for (int ks = 0; ks < 2; ++ks) {
-        Sb[ks][0] = pack_bf16x2(dP[2 * ks][0], dP[2 * ks][1]);
-        Sb[ks][1] = pack_bf16x2(dP[2 * ks][2], dP[2 * ks][3]);
-        Sb[ks][2] = pack_bf16x2(dP[2 * ks + 1][0], dP[2 * ks + 1][1]);
-        Sb[ks][3] = pack_bf16x2(dP[2 * ks + 1][2], dP[2 * ks + 1][3]);
-      }
-      // The dS record of this lane's column (pair e, head g): its 16 keys
-      // (the dQ walk adds dS . K afterwards).
-      if (cvalid) {
-        uint16_t* rec =
-            a.ds_rec + ((((b * a.Lq + q) * a.Hq + (int64_t)h * G + g) * K + k) * 64 + 16 * lg);
-        *reinterpret_cast<u32x4_t*>(rec) = Sb[0];
-        *reinterpret_cast<u32x4_t*>(rec + 8) = Sb[1];
-      }
-    }
-    // this wave's columns of the tiles (columns without a pair or head hold
-    // zeros in dS^T and bf16(w dO)^T, so they add nothing)
-#pragma unroll
-    for (int mt = 0; mt < 4; ++mt)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int key = 16 * mt + 4 * lg + r;
-        tile_put(sm, kKvPt, key, lc, f32_to_bf16(S[mt][r]));
-        tile_put(sm, kKvDs, key, lc, f32_to_bf16(dP[mt][r]));
-      }
-    __syncthreads();
-    // ---- phase 2: keys x dims 32 wave .. + 31, reduction over the columns
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-      u32x4_t bq[2], bw[2];
-#pragma unroll
-      for (int dt = 0; dt < 2; ++dt) {
-        const int dim = 32 * wave + 16 * dt + lj;
-        bq[dt] = tile_read(sm, kKvQt, dim, 4 * ks + lg);
-        bw[dt] = tile_read(sm, kKvWd, dim, 4 * ks + lg);
-      }
-#pragma unroll
-      for (int mt = 0; mt < 4; ++mt) {
-        const u32x4_t ad = tile_read(sm, kKvDs, 16 * mt + lj, 4 * ks + lg);
-        const u32x4_t ap = tile_read(sm, kKvPt, 16 * mt + lj, 4 * ks + lg);
-#pragma unroll
-        for (int dt = 0; dt < 2; ++dt) {
-          dk[mt][dt] = mfma_bf16_16x16x32(ad, bq[dt], dk[mt][dt]);
-          dv[mt][dt] = mfma_bf16_16x16x32(ap, bw[dt], dv[mt][dt]);
+          for (int mt = 0; mt < 2; ++mt) {
+            S[mt] = mfma_bf16_16x16x32(
+                A, mt ? *reinterpret_cast<const u32x4_t*>(kown + 1024 * ks) : kb[ks], S[mt]);
+            dP[mt] = mfma_bf16_16x16x32(
+                D, *reinterpret_cast<const u32x4_t*>(vown + 1024 * (4 * mt + ks)), dP[mt]);
+          }
         }
+      };
+      f32x4_t dP[2][2];
+      float e[2][2][4];        // p = 2^x (STAB: 2^(x - the half's maximum))
+      float* ex = reinterpret_cast<float*>(sm + kDkvExch) + (buf * 2 * kGroups + wave) * 96;
+#pragma unroll
+      for (int ct = 0; ct < 2; ++ct) {
+        f32x4_t S[2];
+        products(ct, S, dP[ct]);
+        float ma[2] = {madd[0], madd[1]};
+        if constexpr (KEEP) {
+          const int32_t v = phalf ? ent[2 * ct + 1] : ent[2 * ct];
+          const int64_t qrow = (row0 + (int64_t)(v & 0xffffff) * a.Hq) / G;  // (b Lq + q) Hkv + h
+          const int8_t* kr = a.keep + (qrow * K + ((v >> 24) & 63)) * 64 + 32 * half + j;
+#pragma unroll
+          for (int mt = 0; mt < 2; ++mt)
+            if (kr[16 * mt] == 0) ma[mt] = ninf;
+        }
+        f32x4_t psum, pd, pmax;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          float x[2];
+#pragma unroll
+          for (int mt = 0; mt < 2; ++mt)
+            x[mt] = alibi(half, mt, r, __builtin_fmaf(S[mt][r], c2, ma[mt]));
+          if constexpr (STAB) {
+            const float m = group16_max(fmaxf(x[0], x[1]));
+            pmax[r] = m;
+            const float mb = m == ninf ? 0.f : m;
+            x[0] -= mb;
+            x[1] -= mb;
+          }
+#pragma unroll
+          for (int mt = 0; mt < 2; ++mt) e[ct][mt][r] = exp2_hw(x[mt]);
+          psum[r] = group16_sum(e[ct][0][r] + e[ct][1][r]);
+          pd[r] = group16_sum(
+              __builtin_fmaf(e[ct][0][r], dP[ct][0][r], e[ct][1][r] * dP[ct][1][r]));
+        }
+        // (the 16 lanes of a group write the same values)
+        float* exc = ex + 16 * ct + 4 * grp;
+        *reinterpret_cast<f32x4_t*>(exc) = psum;
+        *reinterpret_cast<f32x4_t*>(exc + 32) = pd;
+        if constexpr (STAB) *reinterpret_cast<f32x4_t*>(exc + 64) = pmax;
+        __builtin_amdgcn_sched_barrier(0);  // one tile's operands at a time
       }
-    }
-    __syncthreads();
-  }
-  // lane (grp, j) of tile (mt, dt): keys 16 mt + 4 grp + r, dim 32 wave + 16 dt + j
-  float* dkb = a.dk + ((b * a.Lk + c * 64) * a.Hkv + h) * 128;
-  float* dvb = a.dv + ((b * a.Lk + c * 64) * a.Hkv + h) * 128;
-  const int64_t krow = (int64_t)a.Hkv * 128;
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      const float* exo = reinterpret_cast<const float*>(sm + kDkvExch) +
+                         (buf * 2 * kGroups + (wave ^ 1)) * 96 + 4 * grp;
+      u32x4_t dsb[2], wpb[2];  // dS^T and (w P)^T operands: element 4 ct + r
 #pragma unroll
-  for (int mt = 0; mt < 4; ++mt)
+      for (int ct = 0; ct < 2; ++ct) {
+        const int32_t v = phalf ? ent[2 * ct + 1] : ent[2 * ct];
+        const bool have = base + 2 * ct + phalf < e1;
+        const int64_t prow = row0 + (int64_t)(v & 0xffffff) * a.Hq;
+        const int slot = (v >> 24) & 63;
+        // the rows' sums over both halves (the own ones are read back too: they
+        // take no registers across the barrier)
+        const float* exc = ex + 16 * ct + 4 * grp;
+        f32x4_t psum = *reinterpret_cast<const f32x4_t*>(exc);
+        f32x4_t pd = *reinterpret_cast<const f32x4_t*>(exc + 32);
+        const f32x4_t so = *reinterpret_cast<const f32x4_t*>(exo + 16 * ct);
+        const f32x4_t po = *reinterpret_cast<const f32x4_t*>(exo + 32 + 16 * ct);
+        if constexpr (STAB) {
+          const f32x4_t pm = *reinterpret_cast<const f32x4_t*>(exc + 64);
+          const f32x4_t mo = *reinterpret_cast<const f32x4_t*>(exo + 64 + 16 * ct);
 #pragma unroll
-    for (int dt = 0; dt < 2; ++dt)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int64_t off = (int64_t)(16 * mt + 4 * grp + r) * krow + 32 * wave + 16 * dt + j;
-        if (whole) {
-          dkb[off] = dk[mt][dt][r];
-          dvb[off] = dv[mt][dt][r];
+          for (int r = 0; r < 4; ++r) {
+            const float m = fmaxf(pm[r], mo[r]), mb = m == ninf ? 0.f : m;
+            const float f = exp2_hw(pm[r] - mb), fo = exp2_hw(mo[r] - mb);
+            psum[r] = psum[r] * f + so[r] * fo;
+            pd[r] = pd[r] * f + po[r] * fo;
+            e[ct][0][r] *= f;
+            e[ct][1][r] *= f;
+          }
         } else {
-          atomicAdd(dkb + off, dk[mt][dt][r]);
-          atomicAdd(dvb + off, dv[mt][dt][r]);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            psum[r] += so[r];
+            pd[r] += po[r];
+            fine = fine && psum[r] >= 0x1p-64f && psum[r] <= 0x1p64f;
+          }
         }
+        float di[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float inv = psum[r] > 0.f ? rcp_hw(psum[r]) : 0.f;
+          const float wi = have && g4 + r < G ? bf16_to_f32(wraw[ct][r]) * inv : 0.f;
+          di[r] = pd[r] * inv;
+          const float dis = -di[r] * a.scale;
+#pragma unroll
+          for (int mt = 0; mt < 2; ++mt) {
+            const float wp = e[ct][mt][r] * wi;  // w P
+            dP[ct][mt][r] = wp * __builtin_fmaf(dP[ct][mt][r], a.scale, dis);  // dS
+            e[ct][mt][r] = wp;
+          }
+        }
+#pragma unroll
+        for (int mt = 0; mt < 2; ++mt) {
+          dsb[mt][2 * ct] = pack_bf16x2(dP[ct][mt][0], dP[ct][mt][1]);
+          dsb[mt][2 * ct + 1] = pack_bf16x2(dP[ct][mt][2], dP[ct][mt][3]);
+          wpb[mt][2 * ct] = pack_bf16x2(e[ct][mt][0], e[ct][mt][1]);
+          wpb[mt][2 * ct + 1] = pack_bf16x2(e[ct][mt][2], e[ct][mt][3]);
+        }
+        // The dS records (key 32 t + 16 mt + j at 32 t + 2 j + mt) and dW = di;
+        // absent rows write to the sink, so that no branch surrounds the stores.
+        uint16_t* rec = a.ds_rec + ((prow + g4) * K + slot) * 64 + 32 * half + 2 * j;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          uint16_t* dst = have && g4 + r < G ? rec + (int64_t)r * K * 64 : a.sink + 2 * lane;
+          *reinterpret_cast<uint32_t*>(dst) = pack_bf16x2(dP[ct][0][r], dP[ct][1][r]);
+        }
+        const float dj = (j & 2) ? ((j & 1) ? di[3] : di[2]) : ((j & 1) ? di[1] : di[0]);
+        uint16_t* dwp = half == 0 && have && j < 4 && g4 + j < G
+                            ? a.dw + (prow + g4 + j) * K + slot
+                            : a.sink + 2 * lane;
+        *dwp = (uint16_t)f32_to_bf16(dj);
+        __builtin_amdgcn_sched_barrier(0);
       }
+      // row 4 grp + (j >> 2) (+ 16 ct), dims 16 nt + 4 (j & 3): the dim tile
+      // flips bits 5..7
+      const uint32_t rr = lj >> 2;
+      const uint32_t tb = lds_addr(rows) + (uint32_t)buf * 2u * kRowsBytes + 256u * rr +
+                          16u * (rr & 14u) + 16u * (((lj >> 1) ^ rr) & 1u) + 8u * (lj & 1u);
+#pragma unroll
+      for (int nt = 0; nt < 8; ++nt) {
+        const uint32_t ta = tb ^ (32u * nt);
+        const u32x2_t q0 = read_transposed(ta), q1 = read_transposed(ta + 4096u);
+        const u32x2_t o0 = read_transposed(ta + kRowsBytes);
+        const u32x2_t o1 = read_transposed(ta + kRowsBytes + 4096u);
+        const u32x4_t bq = {q0[0], q0[1], q1[0], q1[1]}, bo = {o0[0], o0[1], o1[0], o1[1]};
+#pragma unroll
+        for (int mt = 0; mt < 2; ++mt) {
+          dk[mt][nt] = mfma_bf16_16x16x32(dsb[mt], bq, dk[mt][nt]);
+          dv[mt][nt] = mfma_bf16_16x16x32(wpb[mt], bo, dv[mt][nt]);
+        }
+        if (nt & 1) __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int p = 0; p < kPairs; ++p) ent[p] = entn[p];
+    }
+    return !fine;
+  };
+  // Unstabilised sums lie well inside fp32's range for any |x| well below 64;
+  // a unit with a row outside it (extreme logits) runs again, stabilised.
+  // Keep rows often drop a whole chunk and go there at once, as does a chunk
+  // with no visible key.
+  bool again = KEEP || ~excl == 0ull;
+  if (!again) again = __syncthreads_or(pass(std::integral_constant<bool, false>{}) ? 1 : 0) != 0;
+  if (again) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+#pragma unroll
+    for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+      for (int nt = 0; nt < 8; ++nt) dk[mt][nt] = dv[mt][nt] = zero4();
+    pass(std::integral_constant<bool, true>{});
+  }
+  // The groups' sums through LDS (a tensor at a time, [group][64][128]): lane
+  // (grp, j) of tile (mt, nt) holds keys 16 mt + 4 grp + r of its half, dim
+  // 16 nt + j.
+  float* part = reinterpret_cast<float*>(sm);
+  const int64_t krow = (int64_t)a.Hkv * 128;
+  auto reduce = [&](const f32x4_t (&x)[2][8], float* out) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no DMA is in flight into the region
+    __syncthreads();
+#pragma unroll
+    for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+      for (int nt = 0; nt < 8; ++nt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          part[group * 8192 + (32 * half + 16 * mt + 4 * grp + r) * 128 + 16 * nt + j] =
+              x[mt][nt][r];
+    __syncthreads();
+#pragma unroll 4
+    for (int i = 0; i < 8192 / kDkvThreads; ++i) {
+      const int o = tid + kDkvThreads * i;  // element of [64][128]
+      const float t = (part[o] + part[8192 + o]) + (part[2 * 8192 + o] + part[3 * 8192 + o]);
+      float* dst = out + (int64_t)(o >> 7) * krow + (o & 127);
+      if (whole) *dst = t;
+      else atomicAdd(dst, t);
+    }
+  };
+  reduce(dk, a.dk + ((b * a.Lk + c * 64) * a.Hkv + h) * 128);
+  reduce(dv, a.dv + ((b * a.Lk + c * 64) * a.Hkv + h) * 128);
 }
 
 __global__ void __launch_bounds__(256) fill_zero_i32(int32_t* p, int64_t n) {
@@ -501,8 +612,8 @@ __global__ void __launch_bounds__(256) fill_zero_i32(int32_t* p, int64_t n) {
 struct ListPlan {
   int nqb;
   int64_t n;  // chunks B * Hkv * Ck
-  int64_t count, blkbase, start, ustart, list, records, total;  // byte offsets / size
-  int64_t max_units;
+  int64_t count, blkbase, start, ustart, list, records, sink, total;  // byte offsets / size
+  int64_t max_units, seg;
 };
 
 ListPlan list_plan(int64_t B, int64_t Lq, int64_t Hkv, int64_t K, int64_t Ck, int64_t Hq) {
@@ -522,8 +633,10 @@ ListPlan list_plan(int64_t B, int64_t Lq, int64_t Hkv, int64_t K, int64_t Ck, in
   p.ustart = take((p.n + 1) * 4);
   p.list = take(pairs * 4);
   p.records = take(B * Lq * Hq * K * 64 * 2);  // dS records of the dQ walk
+  p.sink = take(512);
   p.total = o;
-  p.max_units = (pairs + kSegEntries - 1) / kSegEntries + p.n;
+  p.seg = segment_entries(pairs);
+  p.max_units = (pairs + p.seg - 1) / p.seg + p.n;
   return p;
 }
 
@@ -597,19 +710,24 @@ int selected_backward(
   const dim3 lgrid((unsigned)lp.nqb, (unsigned)(batch * kv_heads));
   hipLaunchKernelGGL(list_count_kernel, lgrid, dim3(kListBlock), 0, st, a, count, blkbase, lp.nqb);
   hipLaunchKernelGGL(list_scan_kernel, dim3(1), dim3(1024), 0, st, (const int32_t*)count, lp.n,
-                     start, ustart);
+                     (int)lp.seg, start, ustart);
   a.start = start;
   a.ustart = ustart;
   hipLaunchKernelGGL(list_fill_kernel, lgrid, dim3(kListBlock), 0, st, a,
                      (const int32_t*)blkbase, lp.nqb, list);
   a.list = list;
   a.ds_rec = (uint16_t*)(ws + lp.records);
-  if (slope)
-    hipLaunchKernelGGL(routed_attn_dkv_kernel<true>, dim3((unsigned)lp.max_units), dim3(kThreads),
-                       0, st, a);
-  else
-    hipLaunchKernelGGL(routed_attn_dkv_kernel<false>, dim3((unsigned)lp.max_units), dim3(kThreads),
-                       0, st, a);
+  a.sink = (uint16_t*)(ws + lp.sink);
+  a.seg = (int)lp.seg;
+  auto dkv = slope ? (token_keep ? routed_attn_dkv_kernel<true, true>
+                                 : routed_attn_dkv_kernel<true, false>)
+                   : (token_keep ? routed_attn_dkv_kernel<false, true>
+                                 : routed_attn_dkv_kernel<false, false>);
+  if (hipFuncSetAttribute(reinterpret_cast<const void*>(dkv),
+                          hipFuncAttributeMaxDynamicSharedMemorySize,
+                          (int)kDkvLds) != hipSuccess)
+    return MRSA_ERR_LAUNCH;
+  hipLaunchKernelGGL(dkv, dim3((unsigned)lp.max_units), dim3(kDkvThreads), kDkvLds, st, a);
   const int s2 = mrsa_launch_status();
   if (s2 != MRSA_OK) return s2;
   // dQ: the forward's walk over each query tile's chunks, adding dS . K

@@ -9,6 +9,7 @@ from oracle import mrsa_oracle as O
 pytestmark = pytest.mark.gpu
 
 if torch.cuda.is_available():
+    import mrsa
     from mrsa.route_weights import route_weights_backward
 
 DEV = "cuda:0"
@@ -50,3 +51,52 @@ def test_route_weights_backward_splits_vs_oracle(B, L, C, Hkv, G, K):
     terms = B * L * Hq
     for a, b in ((got[3][1], want[3]), (got[3][0], want[4])):
         assert abs(float(a) - float(b)) <= 1e-5 * terms
+
+
+@pytest.mark.parametrize("Lq,C,Hkv,G,K,keep,alibi,scale", [
+    (1, 1, 1, 1, 1, False, False, 1.0),      # one pair
+    (17, 1, 2, 8, 1, False, True, 1.0),      # 17 pairs of one chunk: one past a round of 16
+    (257, 1, 1, 4, 1, False, False, 1.0),    # one pair past a work unit: two units are added
+    (513, 3, 2, 7, 2, True, False, 1.0),     # keep rows that drop whole chunks
+    (130, 5, 1, 5, 3, False, False, 30.0),   # logits past 2^64: the stabilised second pass
+    (130, 5, 1, 3, 4, True, True, 30.0),
+])
+def test_routed_backward_splits_vs_oracle(Lq, C, Hkv, G, K, keep, alibi, scale):
+    print(f"[gpu-case] routed backward Lq={Lq} C={C} Hkv={Hkv} G={G} K={K} {keep} {alibi}",
+          flush=True)
+    g = torch.Generator().manual_seed(90 + Lq + G)
+    r = lambda *s: torch.randn(*s, generator=g)
+    Hq = Hkv * G
+    q, do = (r(1, Lq, Hq, 128) * scale).bfloat16(), r(1, Lq, Hq, 128).bfloat16()
+    k, v = r(1, C * 64, Hkv, 128).bfloat16(), r(1, C * 64, Hkv, 128).bfloat16()
+    w = torch.rand(1, Lq, Hq, K, generator=g).bfloat16()
+    idx = torch.rand(1, Lq, Hkv, max(C, K), generator=g).topk(K, -1).indices.int()
+    idx[idx >= C] = -1               # (K > C: lists that end early)
+    if C > 1:
+        idx[0, 1, 0, :] = 1          # one chunk in every slot
+    valid = torch.rand(1, C * 64, generator=g) > 0.1
+    if C > 2:
+        valid[0, 64:128] = False     # a chunk with no visible key
+    tk = None
+    if keep:
+        tk = torch.rand(1, Lq, Hkv, K, 64, generator=g) > 0.4
+        tk[0, ::3, :, 0] = False
+        tk = tk.to(torch.int8)
+    slope = torch.rand(Hq, generator=g) if alibi else None
+
+    def grads(fn, dev, dtype, **kw):
+        ins = [t.to(dev, dtype).requires_grad_() for t in (q, k, v, w)]
+        dv = lambda t: None if t is None else t.to(dev)
+        out = fn(*ins, idx.to(dev), dv(valid), token_keep=dv(tk), slope=dv(slope), **kw)
+        out.backward(do.to(dev, dtype))
+        return [t.grad.double().cpu() for t in ins]
+
+    got = grads(lambda *a, **kw: mrsa.HiLS_block_M_head(*a[:5], key_valid=a[5], **kw), DEV,
+                torch.bfloat16)
+    want = grads(O.selected_attention, "cpu", torch.float32)
+    # dS and w P are rounded to bf16 once before the products and the gradients
+    # once after (2^-9 each, independent roundings): 2^-8 of a gradient's norm
+    # each way bounds both
+    for name, a, b in zip(("dq", "dk", "dv", "dw"), got, want):
+        assert torch.isfinite(a).all(), name
+        assert (a - b).norm() <= 2.0 ** -7 * b.norm() + 1e-6, name
