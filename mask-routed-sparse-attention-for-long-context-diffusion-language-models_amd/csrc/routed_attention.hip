@@ -1231,9 +1231,20 @@ __global__ void __launch_bounds__(256) sum_parts_kernel(const float* __restrict_
                                                         const uint16_t* __restrict__ fuse_w) {
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
   for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < n4; e += stride) {
-    f32x4_t s = reinterpret_cast<const f32x4_t*>(partial)[e];
-    for (int p = 1; p < parts; ++p) {
-      const f32x4_t x = reinterpret_cast<const f32x4_t*>(partial)[(int64_t)p * n4 + e];
+    const f32x4_t* src = reinterpret_cast<const f32x4_t*>(partial) + e;
+    f32x4_t s = src[0];
+    int p = 1;
+    for (; p + 4 <= parts; p += 4) {  // four loads in flight, added in order
+      f32x4_t x[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) x[u] = src[(int64_t)(p + u) * n4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) s[i] += x[u][i];
+    }
+    for (; p < parts; ++p) {
+      const f32x4_t x = src[(int64_t)p * n4];
 #pragma unroll
       for (int i = 0; i < 4; ++i) s[i] += x[i];
     }
@@ -1261,6 +1272,10 @@ __global__ void __launch_bounds__(256) fill_neg_inf(float* p, int64_t n) {
 // Lock tries before a tile is deferred (mrsa_set_routed_lock_spin_limit).
 int g_spin_limit = kDefaultSpinLimit;
 
+// Workgroups a short launch is split into: one per CU (a workgroup's registers
+// and LDS take a whole CU, so one more would wait for a second wave of them).
+constexpr int64_t kSplitUnits = 256;
+
 // Largest tile (<= 32 queries, <= 1024 items) whose LDS layout fits, 0 if none.
 int pick_tile(int G, int K, int64_t Ck, bool token, bool keep, bool det) {
   for (int tq = std::min(kMaxTQ, kMaxItems / K); tq >= 4; tq -= 4) {
@@ -1273,8 +1288,18 @@ int pick_tile(int G, int K, int64_t Ck, bool token, bool keep, bool det) {
 template <bool TOKEN, bool KEEP, bool ALIBI = false, bool EXT = false>
 int launch_routed(RaArgs& a, hipStream_t s) {
   if (TOKEN && a.det) return MRSA_ERR_UNSUPPORTED;  // token scoring has no fixed-order walk
-  const int tq = pick_tile(a.G, a.K, a.Ck, TOKEN, KEEP || EXT, a.det != 0);
+  int tq = pick_tile(a.G, a.K, a.Ck, TOKEN, KEEP || EXT, a.det != 0);
   if (tq == 0) return MRSA_ERR_UNSUPPORTED;
+  // A launch that leaves CUs idle takes smaller tiles, as long as they fill at
+  // most one workgroup per CU: a chunk is then read by more tiles, but each
+  // walk is shorter and its prologue, locks and epilogue cover fewer rows.
+  // 4 KV heads, 32 slots, 32 / 16 / 8 / 4 queries per tile: 512 queries 30.8 /
+  // 20.9 / 15.8 (256 workgroups) / 22.3 us, 1024 queries 50.2 / 32.8 (256) /
+  // 40.4 / 62.4, 1536 queries 68.5 (192) / 72.6 / 75.9 / 119.9.
+  for (int t = (tq / 2 + 3) / 4 * 4;
+       t < tq && a.B * a.Hkv * a.parts * ((a.Lq + t - 1) / t) <= kSplitUnits;
+       t = (tq / 2 + 3) / 4 * 4)
+    tq = t;
   a.tq = tq;
   a.ntiles = (a.Lq + tq - 1) / tq;
   a.units = a.B * a.Hkv * a.parts * a.ntiles;

@@ -156,15 +156,9 @@ _SEL_MAX_PARTS = 64
 
 def walk_parts(batch: int, q_len: int, kv_heads: int, kv_len: int, topk: int,
                chunk_size: int = 64) -> int:
-    """Workgroups per (query tile, KV head) walk of the routed attention.
-
-    Long sequences fill the chip with one workgroup per walk.  A short query
-    block (the cached block step: 32 queries, 4 KV heads -> 4 walks of up to
-    1024 chunks) splits each walk into parts of >= 32 steps (at most 512
-    workgroups).  Every part builds the whole walk in its prologue and
-    writes a partial output that the part sum reads back, so more, shorter
-    parts stop paying off: at the cached block step 32 parts take 0.144 ms
-    per block, 16 parts 0.149 ms, 64 parts 0.168 ms.
+    """Parts of >= 32 steps per 32-query walk, at most 512 workgroups: a split
+    for callers that pass ``parts`` themselves.  The launches below choose
+    tiles and parts together (``_split_parts``).
     """
 
     walks = -(-q_len // _SEL_TILE_QUERIES) * kv_heads * batch
@@ -173,6 +167,32 @@ def walk_parts(batch: int, q_len: int, kv_heads: int, kv_len: int, topk: int,
     steps = min(kv_len // chunk_size, min(_SEL_TILE_QUERIES, q_len) * topk)
     parts = min(_SEL_MAX_PARTS, 512 // walks, steps // 32, 65535 // max(batch, 1))
     return max(1, parts)
+
+
+def _split_parts(batch: int, q_len: int, kv_heads: int, kv_len: int, topk: int,
+                 chunk_size: int) -> int:
+    """Walk parts of a launch, beside the kernel's own choice of tile.
+
+    A launch with few walks takes tiles of fewer queries first, down to 4 (the
+    kernel halves them while at most 256 workgroups result); parts of >= 4
+    steps then fill the 256 CUs.  32 queries, 4 KV heads, 32 slots: 19 us at
+    128 chunks (8 parts; 42 us as 4 parts of a 32-query walk), 29 us at 2048
+    chunks (4 parts; 41 us as 32).  A layout past 64 MB (a quarter of the memory-side
+    cache) is bound by its chunk loads, and 128 workgroups reach them: 29 us
+    with 4 parts, 34 us with 8.  There 128 walks take two parts all the same
+    (4 x 32 queries, 256 chunks: 42 us, 49 with one, 45 with four).
+    """
+
+    tile = min(_SEL_TILE_QUERIES, 1024 // topk // 4 * 4)
+    if tile < 4 or q_len == 0 or batch == 0:
+        return 1
+    heads = kv_heads * batch
+    while tile > 4 and -(-q_len // (-(-tile // 8) * 4)) * heads <= 256:
+        tile = -(-tile // 8) * 4
+    walks = -(-q_len // tile) * heads
+    steps = min(kv_len // chunk_size, min(tile, q_len) * topk)
+    units = 128 if heads * kv_len * 512 > 64 << 20 else 256
+    return max(1, min(_SEL_MAX_PARTS, max(units // walks, min(2, 256 // walks)), steps // 4))
 
 
 class RoutedLockTimeout(RuntimeError):
@@ -238,7 +258,7 @@ def selected_attention_launch(
     weights [B, Lq, Hq, K] -> [B, Lq, Hq, D] bf16.
 
     ``parts`` splits each walk over that many workgroups (fp32 partial
-    outputs summed by a second kernel); None picks it with ``walk_parts``.
+    outputs summed by a second kernel); None picks it by the sizes.
     ``token_keep`` [B, Lq, Hkv, K, chunk_size] (nonzero = kept) additionally
     masks the keys of each query's slot k.  ``fuse_local`` [B, Lq, Hq, D] and
     ``fuse_weight`` [B, Lq, Hq] (bf16, both or neither) fold the output
@@ -259,7 +279,7 @@ def selected_attention_launch(
     if sm_scale is None:
         sm_scale = 1.0 / math.sqrt(D)
     if parts is None:
-        parts = walk_parts(B, Lq, Hkv, Lk, K, chunk_size)
+        parts = _split_parts(B, Lq, Hkv, Lk, K, chunk_size)
     parts = int(parts)
     if not 1 <= parts <= _SEL_MAX_PARTS:
         raise ValueError(f"parts must be in [1, {_SEL_MAX_PARTS}], got {parts}")
@@ -431,7 +451,7 @@ def selected_attention_alibi_launch(q, kv_frags, weights, indices, key_valid, ch
     if sm_scale is None:
         sm_scale = 1.0 / math.sqrt(D)
     if parts is None:
-        parts = walk_parts(B, Lq, Hkv, Lk, K, chunk_size)
+        parts = _split_parts(B, Lq, Hkv, Lk, K, chunk_size)
     parts = int(parts)
     if not 1 <= parts <= _SEL_MAX_PARTS:
         raise ValueError(f"parts must be in [1, {_SEL_MAX_PARTS}], got {parts}")

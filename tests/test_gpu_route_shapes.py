@@ -10,6 +10,7 @@ from oracle import mrsa_oracle as O
 pytestmark = pytest.mark.gpu
 
 if torch.cuda.is_available():
+    from mrsa.sparse_attention import kv_fragments, selected_attention_launch
     from mrsa.topk import route_topk_launch
 
 DEV = "cuda:0"
@@ -50,3 +51,32 @@ def test_route_topk_tile_edges_vs_oracle(B, L, C, Hkv, G, topk):
     # the sums' own difference (below 1e-3 at these magnitudes)
     torch.testing.assert_close(sc.cpu().float()[ok], rsc.bfloat16().float()[ok], atol=2e-3,
                                rtol=2.0 ** -8)
+
+
+@pytest.mark.parametrize("B,Lq,C,Hkv,G,K,keep,det", [
+    (1, 1, 40, 4, 7, 32, False, False),    # one query, parts of 4 steps
+    (1, 33, 24, 4, 7, 32, False, False),   # 4-query tiles, the last one partial, parts
+    (2, 64, 30, 2, 7, 16, True, False),    # keep rows, parts
+    (1, 65, 9, 3, 8, 64, False, True),     # fixed order; tiles of 16 at most
+    (1, 641, 11, 4, 7, 32, False, False),  # 16-query tiles: 8 would make 324 workgroups
+    (1, 250, 7, 8, 4, 32, True, False),    # 8-query tiles: 256 workgroups
+    (1, 100, 7, 4, 3, 60, False, False),   # tiles of 16, 8, 4 out of 1024 // 60 = 17 queries
+])
+def test_routed_tiles_and_parts_vs_oracle(B, Lq, C, Hkv, G, K, keep, det):
+    print(f"[gpu-case] routed tiles B={B} Lq={Lq} C={C} Hkv={Hkv} G={G} K={K} {keep} {det}",
+          flush=True)
+    g = torch.Generator().manual_seed(2000 + Lq + C)
+    r = lambda *s: torch.randn(*s, generator=g).bfloat16()
+    q, k, v = r(B, Lq, Hkv * G, 128), r(B, C * 64, Hkv, 128), r(B, C * 64, Hkv, 128)
+    w = torch.softmax(torch.randn(B, Lq, Hkv * G, K, generator=g), -1).bfloat16()
+    idx = torch.rand(B, Lq, Hkv, max(C, K), generator=g).topk(K, -1).indices.int()
+    idx[idx >= C] = -1                    # (K > C: lists that end early)
+    valid = torch.rand(B, C * 64, generator=g) > 0.1
+    tk = (torch.rand(B, Lq, Hkv, K, 64, generator=g) > 0.4).to(torch.int8) if keep else None
+    want = O.selected_attention(q, k, v, w, idx, valid, token_keep=tk)
+    got = selected_attention_launch(
+        q.to(DEV), kv_fragments(k.to(DEV), v.to(DEV)), w.to(DEV), idx.to(DEV), valid.to(DEV), 64,
+        token_keep=None if tk is None else tk.to(DEV), deterministic=det)
+    # w P rounded to bf16 once per term and the output once: 2^-9 of the row's
+    # absolute sum (weights sum to 1, |v| < 5) and of the output
+    torch.testing.assert_close(got.cpu().float(), want, atol=5 * 2.0 ** -9, rtol=2.0 ** -8)
