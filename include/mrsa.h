@@ -550,7 +550,7 @@ int mrsa_local_attention_qf_fwd(const void* q, const void* kv_frags,
  *   grad_q: fp32 [batch, seq_len, q_heads, 128]; grad_k, grad_v: fp32
  *           [batch, seq_len, kv_heads, 128] (every element written)
  *   workspace: 256-byte aligned, mrsa_local_attention_bwd_workspace_bytes
- *           bytes (the operand images of K, V, Q and dO, and per-row lse / D)
+ *           bytes (per-row lse / D, and partial dK / dV of few key blocks)
  * The LSE output carries no gradient (flash-attn's autograd drops it).
  * Rounding points as flash-attn's: P and dS are bf16 matrix operands, every
  * sum is fp32.  Requirements: head_dim 128, 16-byte aligned tensors.

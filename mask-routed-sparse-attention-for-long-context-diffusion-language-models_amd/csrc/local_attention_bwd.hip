@@ -11,23 +11,26 @@
 // autograd drops it).  Rounding points as flash-attn's: P and dS are rounded
 // to bf16 as matrix operands, every sum is fp32.
 //
-// Both passes are one kernel template with the forward's structure: 16
-// matrix columns per wave in registers, 64-row tiles of fragment images
-// streamed through a 2-slot LDS ring by buffer->LDS DMA, one barrier per tile.
-// A slot holds two fragment tiles (mrsa_kv_fragments layout, 32 KB each):
-//   [A: rows x dims images | A': dims x rows images (tiled order)]
-//   [B: rows x dims images | B': dims x rows images (tiled order)]
-//   per tile:  S^T  = A . X1^T,  dP^T = B . X2^T          (32 products)
-//              acc4 += B' . dS^T  (and acc3 += A' . P^T)  (16 or 32 products)
+// Both passes are one kernel template: 16 matrix columns per wave in
+// registers, 64-row tiles of two tensors streamed through a 2-slot LDS ring by
+// buffer->LDS DMA, one barrier per tile.  The rows come as they lie in the
+// tensors, whole 256-byte rows, and serve twice: read along the row (rows x
+// dims) and by gfx950's transposing LDS reads (dims x rows).
+//   per tile:  S^T  = A . X1^T,  dP^T = B . X2^T            (32 products)
+//              acc4 += A^T . dS^T  (and acc3 += B^T . P^T)  (16 or 32 products)
 //  dQ pass   (columns: (query, head); rows: keys):
-//     A = K, B = V, B' = K^T, X1 = Q, X2 = dO  ->  acc4 = dQ / scale
+//     A = K, B = V, X1 = Q, X2 = dO  ->  acc4 = dQ / scale
 //  dK/dV pass (columns: keys; rows: (query, head) pairs, row = query G + head):
-//     A = Q, A' = dO^T, B = dO, B' = Q^T, X1 = K, X2 = V
-//     ->  acc3 = dV, acc4 = dK / scale
+//     A = Q, B = dO, X1 = K, X2 = V  ->  acc3 = dV, acc4 = dK / scale
 // The dQ pass also writes each (query, head) row's lse (log2 units) and D in
-// row order for the dK/dV pass.  The row images of Q and dO come from
-// row_fragments_kernel, which lays out any [B, L, Hkv * G, 128] tensor as a
-// [B, Hkv, L * G] row sequence in the kv_fragments format.
+// row order for the dK/dV pass.
+//
+// Bound: LDS operand reads (64 KB a tile and wave in the dK/dV pass, 4096 of
+// its cycles at 128 B / clock, twice the products').  Operands read 4 (dQ) or 8
+// ahead by explicit order; the dQ pass fits 128 registers and 64 KB of LDS, so
+// that two workgroups share a CU.  28 heads over 4, 16384 queries, window 319:
+// dQ 365 us, dK/dV 443; with pre-transposed images in HBM (four layout
+// launches, 214 us) and 64 KB slots, one workgroup per CU, 473 and 527.
 #include "chunk_tile.h"
 #include "mrsa_device.h"
 
@@ -40,53 +43,36 @@ namespace {
 constexpr int kWaves = 8;
 constexpr int kThreads = 64 * kWaves;
 constexpr int kRing = 2;
-constexpr int kSlotBytes = 65536;     // two fragment tiles
-constexpr int kTileBytes = 32768;
-constexpr int kFragElems = 16384;
-constexpr int kFragPitch = 136;       // LDS row pitch of the layout kernel (elements)
+constexpr int kTileBytes = 16384;     // 64 rows x 256 bytes
+constexpr int kSlotBytes = 2 * kTileBytes;
 constexpr int kMaskTiles = 512;       // inert-key words of the dQ pass kept in LDS
+constexpr int kMaxParts = 8;          // row parts of the dK/dV pass
 
-// Row r of tile c of (b, h): element ((b L + r / G) Hq + h G + r % G) 128 of
-// x / y (G = 1, Hq = Hkv for key rows); rows >= nrows are zero.  Output as
-// mrsa_kv_fragments: x's rows x dims images, then y's dims x rows images.
-__global__ void __launch_bounds__(256)
-    row_fragments_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ y,
-                         int64_t L, int Hq, int Hkv, int G, int64_t NT,
-                         uint16_t* __restrict__ frags) {
-  __shared__ __align__(16) uint16_t xs[64 * kFragPitch];
-  __shared__ __align__(16) uint16_t ys[64 * kFragPitch];
-  const int64_t c = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
-  const int tid = threadIdx.x;
-  const int64_t nrows = L * G;
-  for (int p = tid; p < 1024; p += 256) {
-    const int r = p >> 4, u = p & 15;
-    const int64_t s = c * 64 + r;
-    u32x4_t xv = {0u, 0u, 0u, 0u}, yv = {0u, 0u, 0u, 0u};
-    if (s < nrows) {
-      const int64_t i = s / G, g = s - i * G;
-      const int64_t off = ((b * L + i) * Hq + h * G + g) * 128 + 8 * u;
-      xv = *reinterpret_cast<const u32x4_t*>(x + off);
-      yv = *reinterpret_cast<const u32x4_t*>(y + off);
-    }
-    *reinterpret_cast<u32x4_t*>(xs + r * kFragPitch + 8 * u) = xv;
-    *reinterpret_cast<u32x4_t*>(ys + r * kFragPitch + 8 * u) = yv;
-  }
-  __syncthreads();
-  uint16_t* dst = frags + ((b * Hkv + h) * NT + c) * (int64_t)kFragElems;
-  for (int p = tid; p < 1024; p += 256) {
-    const int i = p >> 6, l = p & 63, j = l & 15, grp = l >> 4;
-    const int mt = i >> 2, kq = i & 3;
-    *reinterpret_cast<u32x4_t*>(dst + 8 * p) =
-        *reinterpret_cast<const u32x4_t*>(xs + (16 * mt + j) * kFragPitch + 32 * kq + 8 * grp);
-    const int nt = i >> 1, kv = i & 1, d = 16 * nt + j;
-    u32x4_t yv;
-#pragma unroll
-    for (int w = 0; w < 4; ++w) {
-      const int r0 = 32 * kv + 16 * (w >> 1) + 4 * grp + 2 * (w & 1);
-      yv[w] = (uint32_t)ys[r0 * kFragPitch + d] | ((uint32_t)ys[(r0 + 1) * kFragPitch + d] << 16);
-    }
-    *reinterpret_cast<u32x4_t*>(dst + 8192 + 8 * p) = yv;
-  }
+typedef short s16x4_t __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) s16x4_t lds_s16x4_t;
+
+// Four 16-bit values of one column out of four LDS rows: lanes 16 g + i of a
+// group point at 8-byte pieces, piece i & 3 of row i >> 2; lane i receives
+// element i of the four rows.
+__device__ __forceinline__ u32x2_t read_transposed(uint32_t addr) {
+  return __builtin_bit_cast(u32x2_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                                         (lds_s16x4_t*)(uintptr_t)addr));
+}
+__device__ __forceinline__ u32x4_t lds_read16(uint32_t addr) {
+  return *(const __attribute__((address_space(3))) u32x4_t*)(uintptr_t)addr;
+}
+
+// Buffer resource of `bytes` bytes at a wave-uniform address, in scalar registers.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t row_rsrc(const uint16_t* at, int bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc((void*)uniform_u64((uint64_t)at), (short)0,
+                                           __builtin_amdgcn_readfirstlane(bytes), 0x00020000);
+}
+
+// Row r's 16-byte part u lies at unit u ^ swizzle(r): 16 rows' reads of one
+// part, and a transposing read's 8 rows x 2 parts, meet 16 different units of
+// the 64 banks.
+__device__ __forceinline__ uint32_t swizzle(uint32_t r) {
+  return 2u * (r & 7u) + ((r >> 3) & 1u);
 }
 
 struct BwdArgs {
@@ -97,15 +83,16 @@ struct BwdArgs {
   const uint16_t* dout;
   const float* lse;           // [B, L, Hq] natural log
   const uint8_t* key_valid;
-  const uint16_t* fa;         // per pass: the A | A' fragment sequence
-  const uint16_t* fb;         // per pass: the B | B' fragment sequence
   int64_t B, L;
   int Hq, Hkv, G;
   int64_t W;
   int64_t inert_chunk;
   float scale, scale_log2;
-  float* lse_rows;            // [B, Hkv, L G] log2 units (written by the dQ pass)
-  float* d_rows;              // [B, Hkv, L G]
+  int64_t row_pitch;          // L G rounded up to 64
+  float* lse_rows;            // [B, Hkv, row_pitch] log2 units (written by the dQ pass)
+  float* d_rows;              // [B, Hkv, row_pitch]
+  int parts;                  // row parts of the dK/dV pass
+  float* partial;             // parts > 1: [parts, 2 (dk, dv), B, L, Hkv, 128] fp32
   float* dq;                  // [B, L, Hq, 128] fp32
   float* dk;                  // [B, L, Hkv, 128] fp32
   float* dv;
@@ -132,42 +119,9 @@ __device__ __forceinline__ bool key_inert(const BwdArgs& a, int64_t b, int64_t j
   return a.inert_chunk > 0 && (j + 1) % a.inert_chunk == 0;
 }
 
-// The 16 S^T accumulator values of a lane packed as the B operand of a
-// dims x rows product (reduction index 8 grp + e of step ks = row 32 ks + 16
-// (e >> 2) + 4 grp + (e & 3), the tiled order of the fragments).
-__device__ __forceinline__ void pack_rows(const f32x4_t (&X)[4], u32x4_t (&Xb)[2]) {
-#pragma unroll
-  for (int jj = 0; jj < 2; ++jj) {
-    Xb[jj][0] = pack_bf16x2(X[2 * jj][0], X[2 * jj][1]);
-    Xb[jj][1] = pack_bf16x2(X[2 * jj][2], X[2 * jj][3]);
-    Xb[jj][2] = pack_bf16x2(X[2 * jj + 1][0], X[2 * jj + 1][1]);
-    Xb[jj][3] = pack_bf16x2(X[2 * jj + 1][2], X[2 * jj + 1][3]);
-  }
-}
-
-// acc += (dims x rows images at laddr + OFF) . Xb
-template <int OFF>
-__device__ __forceinline__ void dims_rows_product(uint32_t laddr, const u32x4_t (&Xb)[2],
-                                                  f32x4_t (&acc)[8]) {
-  constexpr int kD = 8;
-  u32x4_t vb[16];
-  static_for<kD>([&](auto oc) {
-    constexpr int o = decltype(oc)::value;
-    vb[o] = lds_read_b128<OFF + (2 * (o & 7) + (o >> 3)) * 1024>(laddr);
-  });
-  static_for<16>([&](auto oc) {
-    constexpr int o = decltype(oc)::value;
-    lds_wait<(15 - o < kD - 1 ? 15 - o : kD - 1)>(vb[o]);
-    acc[o & 7] = mfma_bf16_16x16x32(vb[o], Xb[o >> 3], acc[o & 7]);
-    if constexpr (o + kD < 16)
-      vb[o + kD] = lds_read_b128<OFF + (2 * ((o + kD) & 7) + ((o + kD) >> 3)) * 1024>(laddr);
-    __builtin_amdgcn_sched_barrier(0);
-  });
-}
-
 template <bool DKV>
-__global__ void __launch_bounds__(kThreads, 1) local_bwd_kernel(BwdArgs a) {
-  extern __shared__ __align__(16) unsigned char smem[];
+__global__ void __launch_bounds__(kThreads, DKV ? 2 : 4) local_bwd_kernel(BwdArgs a) {
+  extern __shared__ __align__(256) unsigned char smem[];
   unsigned char* ring = smem;
   uint64_t* inert_tab = reinterpret_cast<uint64_t*>(smem + kRing * kSlotBytes);  // [kMaskTiles]
 
@@ -182,7 +136,9 @@ __global__ void __launch_bounds__(kThreads, 1) local_bwd_kernel(BwdArgs a) {
     const int64_t x = lin % 8, q8 = total / 8, r8 = total % 8;
     lin = x * q8 + min(x, r8) + lin / 8;
   }
-  const int64_t blk = lin % nx;
+  const int parts = DKV ? a.parts : 1;
+  const int part = (int)(lin % parts);
+  const int64_t blk = lin % nx / parts;
   const int h = (int)((lin / nx) % gridDim.y);
   const int64_t b = lin / (nx * gridDim.y);
   const int G = a.G, Hq = a.Hq;
@@ -226,7 +182,7 @@ __global__ void __launch_bounds__(kThreads, 1) local_bwd_kernel(BwdArgs a) {
     const float lse = cok ? a.lse[(b * L + cq) * Hq + (int64_t)h * G + cg] : 0.f;
     lse2_c = lse * kLog2e;
     if (cok && grp == 0) {
-      const int64_t ridx = (b * a.Hkv + h) * (L * G) + cq * G + cg;
+      const int64_t ridx = (b * a.Hkv + h) * a.row_pitch + cq * G + cg;
       a.lse_rows[ridx] = lse2_c;
       a.d_rows[ridx] = d_c;
     }
@@ -253,46 +209,82 @@ __global__ void __launch_bounds__(kThreads, 1) local_bwd_kernel(BwdArgs a) {
     rhi = 0;
   }
 
-  // ---- the workgroup's row tiles: the union of its columns' windows
+  // ---- the workgroup's row tiles: the union of its columns' windows (of
+  // which a part takes its share), and this wave's rows
   int64_t lo_all, hi_all;
+  int64_t wlo = 0, whi = -1;   // rows some column of the wave sees
+  int64_t flo = 0, fhi = -1;   // rows all of them see
   if constexpr (!DKV) {
     const int QB = 128 / G;
     const int64_t q0 = blk * QB, q1 = min(q0 + QB, L) - 1;
     lo_all = max(q0 - W, (int64_t)0);
     hi_all = min(q1 + W, L - 1);
+    const int64_t a0 = q0 + 16 * wave / G, a1 = min(q0 + (16 * wave + 15) / G, q1);
+    if (16 * wave < QB * G && a0 < L) {
+      wlo = max(a0 - W, (int64_t)0);
+      whi = min(a1 + W, L - 1);
+      flo = max(a1 - W, (int64_t)0);
+      fhi = min(a0 + W, L - 1);
+    }
   } else {
     const int64_t j0 = blk * 128, j1 = min(j0 + 128, L) - 1;
     lo_all = G * max(j0 - W, (int64_t)0);
     hi_all = G * min(j1 + W, L - 1) + G - 1;
+    const int64_t a0 = j0 + 16 * wave, a1 = min(a0 + 15, L - 1);
+    if (a0 < L) {
+      wlo = G * max(a0 - W, (int64_t)0);
+      whi = G * min(a1 + W, L - 1) + G - 1;
+      flo = G * max(a1 - W, (int64_t)0);
+      fhi = G * min(a0 + W, L - 1) + G - 1;
+    }
   }
-  const int64_t t0 = lo_all / 64, t1 = hi_all / 64;
-  const int ntiles = (int)max(t1 - t0 + 1, (int64_t)0);
-  const int64_t NT = (nrows + 63) / 64;
+  const int64_t tall = hi_all / 64 - lo_all / 64 + 1;
+  const int64_t t0 = lo_all / 64 + tall * part / parts;
+  const int ntiles = (int)(lo_all / 64 + tall * (part + 1) / parts - t0);
   const bool tab = !DKV && ntiles <= kMaskTiles;
 
-  const __amdgpu_buffer_rsrc_t ras = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<uint16_t*>(a.fa + (b * a.Hkv + h) * NT * (int64_t)kFragElems), (short)0,
-      (int)(uint32_t)(NT * kTileBytes), 0x00020000);
-  const __amdgpu_buffer_rsrc_t rbs = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<uint16_t*>(a.fb + (b * a.Hkv + h) * NT * (int64_t)kFragElems), (short)0,
-      (int)(uint32_t)(NT * kTileBytes), 0x00020000);
-  const uint32_t dma_lane = 16u * lane;
-  // Tile t into slot s: each wave 4 images of A|A' and 4 of B|B' (the dQ
-  // pass reads no A', the images of waves 4..7).
-  auto issue_tile = [&](int64_t t, int s) {
-    unsigned char* da = ring + s * kSlotBytes + (4 * wave) * 1024;
-    unsigned char* db = da + kTileBytes;
-    const uint32_t src = (uint32_t)t * (uint32_t)kTileBytes + (uint32_t)(4 * wave) * 1024u;
-    if (DKV || wave < 4) {
+  // ---- the stream: row s of (b, h) is row (s / RG) RH + h RG + s % RG of the
+  // tensors.  Instruction n of a wave fills rows 8 wave + 4 n + (lane >> 4) of
+  // the tile; rows past the last repeat it (nothing sees them).
+  const int RG = DKV ? G : 1, RH = DKV ? Hq : a.Hkv;
+  const uint16_t* const xa = (DKV ? a.q : a.k) + (b * L * RH + (int64_t)h * RG) * 128;
+  const uint16_t* const xb = (DKV ? a.dout : a.v) + (b * L * RH + (int64_t)h * RG) * 128;
+  int ri[2], rg[2];            // position and head of each instruction's first row
 #pragma unroll
-      for (int u = 0; u < 4; ++u)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(ras, (lds_void_t*)(da + u * 1024), 16, dma_lane,
-                                                 src + 1024u * u, 0, 0);
+  for (int n = 0; n < 2; ++n) {
+    const int s = __builtin_amdgcn_readfirstlane((int)(t0 * 64) + 8 * wave + 4 * n);
+    ri[n] = s / RG;
+    rg[n] = s % RG;
+  }
+  const int step_i = 64 / RG, step_g = 64 % RG;
+  // The next tile into slot s.
+  auto issue_tile = [&](int s) {
+    unsigned char* dst = ring + s * kSlotBytes + 2048 * wave;
+#pragma unroll
+    for (int n = 0; n < 2; ++n) {
+      const int last = (int)L - 1;
+      const int i0 = __builtin_amdgcn_readfirstlane(min(ri[n], last));
+      const int v = rg[n] + grp;
+      const int di = (v >= RG) + (v >= 2 * RG) + (v >= 3 * RG);
+      const bool in = ri[n] + di <= last;
+      const uint32_t row = in ? (uint32_t)di * (uint32_t)RH + (uint32_t)(v - di * RG)
+                              : (uint32_t)(last - i0) * (uint32_t)RH + (uint32_t)(RG - 1);
+      const uint32_t off = 256u * row + 16u * ((uint32_t)col ^ swizzle(8u * wave + 4u * n + grp));
+      const int64_t left = ((int64_t)(last - i0) * RH + RG) * 256;
+      const int bytes = left < 0xfffffff0ll ? (int)(uint32_t)left : -16;
+      const __amdgpu_buffer_rsrc_t ra = row_rsrc(xa + (int64_t)i0 * RH * 128, bytes);
+      const __amdgpu_buffer_rsrc_t rb = row_rsrc(xb + (int64_t)i0 * RH * 128, bytes);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_void_t*)(dst + 1024 * n), 16, off, 0, 0,
+                                               0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          rb, (lds_void_t*)(dst + kTileBytes + 1024 * n), 16, off, 0, 0, 0);
+      ri[n] += step_i;
+      rg[n] += step_g;
+      if (rg[n] >= RG) {
+        rg[n] -= RG;
+        ++ri[n];
+      }
     }
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rbs, (lds_void_t*)(db + u * 1024), 16, dma_lane,
-                                               src + 1024u * u, 0, 0);
   };
   if constexpr (!DKV) {
     if (tab)
@@ -306,7 +298,7 @@ __global__ void __launch_bounds__(kThreads, 1) local_bwd_kernel(BwdArgs a) {
     asm volatile("" : "+v"(X1[j]));
     asm volatile("" : "+v"(X2[j]));
   }
-  if (ntiles > 0) issue_tile(t0, 0);
+  if (ntiles > 0) issue_tile(0);
 
   f32x4_t acc3[8], acc4[8];
 #pragma unroll
@@ -315,65 +307,129 @@ __global__ void __launch_bounds__(kThreads, 1) local_bwd_kernel(BwdArgs a) {
     acc4[td] = zero4();
   }
   const float c = a.scale_log2;
+  // This lane's operand rows (row col, part 4 kq + grp: kq flips bits 6, 7)
+  // and transposed reads (row 4 grp + (col >> 2), dims 4 (col & 3) ..: the dim
+  // tile flips bits 5..7), within a slot.
+  const bool any = rhi >= rlo;
+  const uint32_t span = (uint32_t)(rhi - rlo);
+  const uint32_t arow = 256u * col + 16u * ((uint32_t)grp ^ swizzle(col));
+  const uint32_t rt = 4u * grp + (col >> 2);
+  const uint32_t trow = 256u * rt + 16u * (((col >> 1) & 1u) ^ swizzle(rt)) + 8u * (col & 1u);
 
   for (int t = 0; t < ntiles; ++t) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     const int64_t r0 = (t0 + t) * 64;
-    // per-row values of the dK/dV pass (row-ordered lse and D, clamped
-    // rows), issued before the next tile's DMA so that their wait does not
-    // wait for it
-    float lse2_r[4][4], d_r[4][4];
+    const bool seen = r0 + 63 >= wlo && r0 <= whi;  // wave-uniform
+    // per-row values of the dK/dV pass, issued before the next tile's DMA so
+    // that their wait does not wait for it
+    f32x4_t lse2_r[4], d_r[4];
     if constexpr (DKV) {
-      const int64_t rb = (b * a.Hkv + h) * nrows;
+      const int64_t rb = (b * a.Hkv + h) * a.row_pitch + r0 + 4 * grp;
 #pragma unroll
-      for (int mt = 0; mt < 4; ++mt)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int64_t rr = min(r0 + 16 * mt + 4 * grp + r, nrows - 1);
-          lse2_r[mt][r] = a.lse_rows[rb + rr];
-          d_r[mt][r] = a.d_rows[rb + rr];
-        }
+      for (int mt = 0; mt < 4; ++mt) {
+        lse2_r[mt] = *reinterpret_cast<const f32x4_t*>(a.lse_rows + rb + 16 * mt);
+        d_r[mt] = *reinterpret_cast<const f32x4_t*>(a.d_rows + rb + 16 * mt);
+      }
     }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    if (t + 1 < ntiles) issue_tile(t0 + t + 1, (t + 1) % kRing);
+    if (t + 1 < ntiles) issue_tile((t + 1) % kRing);
+    asm volatile("" ::: "memory");
     const uint32_t sbase = lds_addr(ring + (t % kRing) * kSlotBytes);
-    const uint32_t laddr = sbase + 16u * lane;
     uint64_t inert = 0ull;
     if constexpr (!DKV) inert = uniform_u64(tab ? lds_read_u64(lds_addr(&inert_tab[t]))
                                                 : inert_bits(a, b, t0 + t));
-
-    f32x4_t S[4], dP[4];
-    qk_frag<8>(laddr, X1, S);
-    qk_frag<8>(laddr + kTileBytes, X2, dP);
+    if (!seen) continue;
 
     // P and dS of the visible rows: row r0 + 16 mt + 4 grp + r lies in
-    // [rlo, rhi] (one unsigned compare); the dQ pass drops inert key rows
-    // from dS (their k' = 0 adds nothing to dQ).
-    const int64_t rel = r0 + 4 * grp - rlo;
-    const uint64_t span = (uint64_t)(rhi - rlo);
-    const uint64_t msh = inert >> (4 * grp);
+    // [rlo, rhi] (one unsigned compare; none where every column sees the whole
+    // tile); the dQ pass drops inert key rows from dS (their k' = 0 adds
+    // nothing).
+    const int rel = (int)r0 + 4 * grp - (int)rlo;
+    const bool plain = r0 >= flo && r0 + 63 <= fhi && inert == 0;  // wave-uniform
+    const uint32_t at = sbase + arow, tt = sbase + trow;
+    auto rows32 = [&](auto hc) {
+      constexpr int hh = decltype(hc)::value;
+      constexpr int kRead = DKV ? 8 : 4;
+      f32x4_t S[2], dP[2];
+      S[0] = S[1] = dP[0] = dP[1] = zero4();
+      // product o: part kq = o >> 2, S (o & 2 == 0) or dP, rows 16 (o & 1) ..;
+      // kRead operand reads in flight
+      auto operand = [&](int o) {
+        return lds_read16((at ^ (64u * (o >> 2))) + 4096u * (2 * hh + (o & 1)) +
+                          ((o & 2) ? (uint32_t)kTileBytes : 0u));
+      };
+      u32x4_t x[16];
 #pragma unroll
-    for (int mt = 0; mt < 4; ++mt)
+      for (int o = 0; o < kRead; ++o) x[o] = operand(o);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const bool vis = rhi >= rlo && (uint64_t)(rel + 16 * mt + r) <= span;
-        const float l2 = DKV ? lse2_r[mt][r] : lse2_c;
-        const float dd = DKV ? d_r[mt][r] : d_c;
-        const float p = vis ? exp2_hw(__builtin_fmaf(S[mt][r], c, -l2)) : 0.f;
-        const bool ds_ok = vis && (DKV || !((msh >> (16 * mt + r)) & 1ull));
-        S[mt][r] = p;
-        dP[mt][r] = ds_ok ? p * (dP[mt][r] - dd) : 0.f;
+      for (int o = 0; o < 16; ++o) {
+        if (o & 2)
+          dP[o & 1] = mfma_bf16_16x16x32(x[o], X2[o >> 2], dP[o & 1]);
+        else
+          S[o & 1] = mfma_bf16_16x16x32(x[o], X1[o >> 2], S[o & 1]);
+        if (o + kRead < 16) x[o + kRead] = operand(o + kRead);
+        __builtin_amdgcn_sched_barrier(0);
       }
-    u32x4_t Sb[2];
-    pack_rows(dP, Sb);
-    dims_rows_product<kTileBytes + 16384>(laddr, Sb, acc4);
-    if constexpr (DKV) {
-      u32x4_t Pb[2];
-      pack_rows(S, Pb);
-      dims_rows_product<16384>(laddr, Pb, acc3);
-    }
+#pragma unroll
+      for (int m = 0; m < 2; ++m)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float l2 = DKV ? lse2_r[2 * hh + m][r] : lse2_c;
+          const float dd = DKV ? d_r[2 * hh + m][r] : d_c;
+          const float p = exp2_hw(__builtin_fmaf(S[m][r], c, -l2));
+          S[m][r] = p;
+          dP[m][r] = p * (dP[m][r] - dd);
+        }
+      const uint32_t dead = (uint32_t)(inert >> (32 * hh)) >> (4 * grp);
+      if (!plain) {
+#pragma unroll
+        for (int m = 0; m < 2; ++m)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const bool vis = any & ((uint32_t)(rel + 32 * hh + 16 * m + r) <= span);
+            if constexpr (DKV) S[m][r] = vis ? S[m][r] : 0.f;
+            const bool live = DKV ? vis : vis & (((dead >> (16 * m + r)) & 1u) == 0u);
+            dP[m][r] = live ? dP[m][r] : 0.f;
+          }
+      }
+      u32x4_t Pb, Sb;  // the B operands: element 4 m + r is row 32 hh + 16 m + 4 grp + r
+#pragma unroll
+      for (int m = 0; m < 2; ++m) {
+        Sb[2 * m] = pack_bf16x2(dP[m][0], dP[m][1]);
+        Sb[2 * m + 1] = pack_bf16x2(dP[m][2], dP[m][3]);
+        if constexpr (DKV) {
+          Pb[2 * m] = pack_bf16x2(S[m][0], S[m][1]);
+          Pb[2 * m + 1] = pack_bf16x2(S[m][2], S[m][3]);
+        }
+      }
+      // product o: dims 16 (o >> DKV) .., of A^T . dS^T or (o & 1) B^T . P^T;
+      // kRead / 2 operands (two reads each) in flight
+      constexpr int N = DKV ? 16 : 8, kT = kRead / 2;
+      auto transposed = [&](int o) {
+        const uint32_t ad = (tt ^ (32u * (DKV ? o >> 1 : o))) + 8192u * hh +
+                            (DKV && (o & 1) ? (uint32_t)kTileBytes : 0u);
+        const u32x2_t y0 = read_transposed(ad), y1 = read_transposed(ad + 4096u);
+        return u32x4_t{y0[0], y0[1], y1[0], y1[1]};
+      };
+      u32x4_t y[N];
+#pragma unroll
+      for (int o = 0; o < kT; ++o) y[o] = transposed(o);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int o = 0; o < N; ++o) {
+        if (DKV && (o & 1))
+          acc3[o >> 1] = mfma_bf16_16x16x32(y[o], Pb, acc3[o >> 1]);
+        else
+          acc4[DKV ? o >> 1 : o] = mfma_bf16_16x16x32(y[o], Sb, acc4[DKV ? o >> 1 : o]);
+        if (o + kT < N) y[o + kT] = transposed(o + kT);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
+    rows32(std::integral_constant<int, 0>{});
+    rows32(std::integral_constant<int, 1>{});
   }
 
   // ---- outputs (fp32): the lane holds dims 16 td + 4 grp .. + 3 of its column
@@ -389,8 +445,10 @@ __global__ void __launch_bounds__(kThreads, 1) local_bwd_kernel(BwdArgs a) {
     }
   } else {
     const bool dead = key_inert(a, b, cj);  // dk = dK' m, dv = dV' m
-    float* dk = a.dk + ((b * L + cj) * a.Hkv + h) * 128;
-    float* dv = a.dv + ((b * L + cj) * a.Hkv + h) * 128;
+    const int64_t n = a.B * L * a.Hkv * 128;
+    const int64_t at = ((b * L + cj) * a.Hkv + h) * 128;
+    float* dk = (parts > 1 ? a.partial + (int64_t)part * 2 * n : a.dk) + at;
+    float* dv = (parts > 1 ? a.partial + ((int64_t)part * 2 + 1) * n : a.dv) + at;
 #pragma unroll
     for (int td = 0; td < 8; ++td) {
       f32x4_t ok = acc4[td], ov = acc3[td];
@@ -405,32 +463,71 @@ __global__ void __launch_bounds__(kThreads, 1) local_bwd_kernel(BwdArgs a) {
   }
 }
 
+// dk and dv of a dK/dV pass in parts: n4 vectors of each, added in order.
+__global__ void __launch_bounds__(256)
+    local_bwd_sum_kernel(const float* __restrict__ partial, int parts, int64_t n4,
+                         float* __restrict__ dk, float* __restrict__ dv) {
+  const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (e >= 2 * n4) return;
+  const f32x4_t* src = reinterpret_cast<const f32x4_t*>(partial) + e;
+  f32x4_t s = src[0];
+  for (int p = 1; p < parts; ++p) {
+    const f32x4_t x = src[(int64_t)p * 2 * n4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) s[i] += x[i];
+  }
+  reinterpret_cast<f32x4_t*>(e < n4 ? dk : dv)[e < n4 ? e : e - n4] = s;
+}
+
 struct BwdPlan {
-  int64_t ntk, ntr;               // key tiles, row tiles per (batch, KV head)
-  size_t kv, vk, qd, dq, lse, d;  // workspace offsets
+  int64_t row_pitch;        // L G rounded up to 64
+  int max_parts;
+  size_t lse, d, partial;   // workspace offsets
   size_t total;
 };
 
+int64_t key_blocks(int64_t B, int64_t L, int64_t Hkv) { return B * Hkv * ((L + 127) / 128); }
+
 BwdPlan bwd_plan(int64_t B, int64_t L, int64_t Hkv, int64_t G) {
   BwdPlan p;
-  p.ntk = (L + 63) / 64;
-  p.ntr = (L * G + 63) / 64;
+  p.row_pitch = (L * G + 63) / 64 * 64;
+  const int64_t units = std::max<int64_t>(key_blocks(B, L, Hkv), 1);
+  p.max_parts = (int)std::clamp<int64_t>(1024 / units, 1, kMaxParts);
   size_t o = 0;
   auto take = [&](size_t n) {
     const size_t at = o;
     o += (n + 255) & ~(size_t)255;
     return at;
   };
-  const size_t kf = (size_t)(B * Hkv * p.ntk) * kTileBytes;
-  const size_t rf = (size_t)(B * Hkv * p.ntr) * kTileBytes;
-  p.kv = take(kf);
-  p.vk = take(kf);
-  p.qd = take(rf);
-  p.dq = take(rf);
-  p.lse = take((size_t)(B * Hkv * L * G) * 4);
-  p.d = take((size_t)(B * Hkv * L * G) * 4);
+  p.lse = take((size_t)(B * Hkv * p.row_pitch) * 4);
+  p.d = take((size_t)(B * Hkv * p.row_pitch) * 4);
+  p.partial = take(p.max_parts > 1 ? (size_t)(p.max_parts * B * L * Hkv) * 1024 : 0);
   p.total = o;
   return p;
+}
+
+// Row parts of the dK/dV pass.  A workgroup (128 keys) has a CU to itself, so
+// the launch takes ceil(units parts / 256) rounds of its tiles / parts, each
+// with about 6 tiles' time around the loop; a part writes and reads back 2 KB
+// per key row, a tile's time (2.5 us) for 10 MB.
+// 5003 keys, window 1280 (160 workgroups of 295 tiles): 543 us in 3 parts with
+// 13 for their sum, 780 whole (in the pre-transposed form; 1.2 times less in
+// this one at whole rounds).
+int pick_parts(const BwdPlan& p, int64_t B, int64_t L, int64_t Hkv, int64_t G, int64_t W) {
+  const int64_t units = key_blocks(B, L, Hkv);
+  const int64_t tiles = (G * std::min(L, 128 + 2 * std::min(W, L)) + 63) / 64;
+  int best = 1;
+  double least = 0.;
+  for (int n = 1; n <= p.max_parts && (n == 1 || tiles / n >= 4); ++n) {
+    const double rounds = (double)((units * n + 255) / 256);
+    const double cost = rounds * ((double)((tiles + n - 1) / n) + 6.) +
+                        (n > 1 ? 2. + n * (double)(B * L * Hkv) * 2048. / 1e7 : 0.);
+    if (n == 1 || cost < least) {
+      least = cost;
+      best = n;
+    }
+  }
+  return best;
 }
 
 }  // namespace
@@ -458,7 +555,7 @@ extern "C" int mrsa_local_attention_bwd(const void* q, const void* k, const void
   if (head_dim != 128) return MRSA_ERR_UNSUPPORTED;
   const int64_t G = q_heads / kv_heads;
   if (G > 128 || kv_heads > 65535 || batch > 65535) return MRSA_ERR_UNSUPPORTED;
-  // fragment sequences are addressed with 32-bit byte offsets
+  // rows and tiles are counted in 32 bits
   if ((seq_len * G + 63) / 64 >= 131072) return MRSA_ERR_UNSUPPORTED;
   if (!q || !k || !v || !out || !lse || !grad_out || !grad_q || !grad_k || !grad_v || !workspace)
     return MRSA_ERR_INVALID_ARGUMENT;
@@ -469,32 +566,13 @@ extern "C" int mrsa_local_attention_bwd(const void* q, const void* k, const void
   if (workspace_bytes < (int64_t)p.total || (uintptr_t)workspace % 256 != 0)
     return MRSA_ERR_INVALID_ARGUMENT;
   char* ws = (char*)workspace;
-  uint16_t* f_kv = (uint16_t*)(ws + p.kv);
-  uint16_t* f_vk = (uint16_t*)(ws + p.vk);
-  uint16_t* f_qd = (uint16_t*)(ws + p.qd);
-  uint16_t* f_dq = (uint16_t*)(ws + p.dq);
   hipStream_t s = (hipStream_t)stream;
-  const uint16_t *q16 = (const uint16_t*)q, *k16 = (const uint16_t*)k, *v16 = (const uint16_t*)v,
-                 *o16 = (const uint16_t*)out, *do16 = (const uint16_t*)grad_out;
-  const dim3 kgrid((unsigned)p.ntk, (unsigned)kv_heads, (unsigned)batch);
-  const dim3 rgrid((unsigned)p.ntr, (unsigned)kv_heads, (unsigned)batch);
-  hipLaunchKernelGGL(row_fragments_kernel, kgrid, dim3(256), 0, s, k16, v16, seq_len,
-                     (int)kv_heads, (int)kv_heads, 1, p.ntk, f_kv);
-  hipLaunchKernelGGL(row_fragments_kernel, kgrid, dim3(256), 0, s, v16, k16, seq_len,
-                     (int)kv_heads, (int)kv_heads, 1, p.ntk, f_vk);
-  hipLaunchKernelGGL(row_fragments_kernel, rgrid, dim3(256), 0, s, q16, do16, seq_len,
-                     (int)q_heads, (int)kv_heads, (int)G, p.ntr, f_qd);
-  hipLaunchKernelGGL(row_fragments_kernel, rgrid, dim3(256), 0, s, do16, q16, seq_len,
-                     (int)q_heads, (int)kv_heads, (int)G, p.ntr, f_dq);
-  int st = mrsa_launch_status();
-  if (st != MRSA_OK) return st;
-
   BwdArgs a;
-  a.q = q16;
-  a.k = k16;
-  a.v = v16;
-  a.out = o16;
-  a.dout = do16;
+  a.q = (const uint16_t*)q;
+  a.k = (const uint16_t*)k;
+  a.v = (const uint16_t*)v;
+  a.out = (const uint16_t*)out;
+  a.dout = (const uint16_t*)grad_out;
   a.lse = lse;
   a.key_valid = key_valid;
   a.B = batch;
@@ -506,15 +584,15 @@ extern "C" int mrsa_local_attention_bwd(const void* q, const void* k, const void
   a.inert_chunk = inert_chunk;
   a.scale = sm_scale;
   a.scale_log2 = sm_scale * kLog2e;
+  a.row_pitch = p.row_pitch;
+  a.parts = pick_parts(p, batch, seq_len, kv_heads, G, window);
+  a.partial = (float*)(ws + p.partial);
   a.lse_rows = (float*)(ws + p.lse);
   a.d_rows = (float*)(ws + p.d);
   a.dq = grad_q;
   a.dk = grad_k;
   a.dv = grad_v;
   const size_t smem = (size_t)kRing * kSlotBytes + kMaskTiles * 8;
-  // dQ pass: columns (query, head), rows = keys: A = K, B = V, B' = K^T
-  a.fa = f_kv;
-  a.fb = f_vk;
   if (hipFuncSetAttribute(reinterpret_cast<const void*>(local_bwd_kernel<false>),
                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess)
     return MRSA_ERR_LAUNCH;
@@ -522,16 +600,19 @@ extern "C" int mrsa_local_attention_bwd(const void* q, const void* k, const void
   hipLaunchKernelGGL(local_bwd_kernel<false>,
                      dim3((unsigned)((seq_len + QB - 1) / QB), (unsigned)kv_heads, (unsigned)batch),
                      dim3(kThreads), smem, s, a);
-  st = mrsa_launch_status();
+  int st = mrsa_launch_status();
   if (st != MRSA_OK) return st;
-  // dK/dV pass: columns = keys, rows = (query, head): A = Q, A' = dO^T, B = dO, B' = Q^T
-  a.fa = f_qd;
-  a.fb = f_dq;
   if (hipFuncSetAttribute(reinterpret_cast<const void*>(local_bwd_kernel<true>),
                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess)
     return MRSA_ERR_LAUNCH;
   hipLaunchKernelGGL(local_bwd_kernel<true>,
-                     dim3((unsigned)((seq_len + 127) / 128), (unsigned)kv_heads, (unsigned)batch),
+                     dim3((unsigned)((seq_len + 127) / 128 * a.parts), (unsigned)kv_heads,
+                          (unsigned)batch),
                      dim3(kThreads), smem, s, a);
+  st = mrsa_launch_status();
+  if (st != MRSA_OK || a.parts == 1) return st;
+  const int64_t n4 = batch * seq_len * kv_heads * 32;
+  hipLaunchKernelGGL(local_bwd_sum_kernel, dim3((unsigned)((2 * n4 + 255) / 256)), dim3(256), 0, s,
+                     a.partial, a.parts, n4, grad_k, grad_v);
   return mrsa_launch_status();
 }

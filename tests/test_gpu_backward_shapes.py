@@ -100,3 +100,60 @@ def test_routed_backward_splits_vs_oracle(Lq, C, Hkv, G, K, keep, alibi, scale):
     for name, a, b in zip(("dq", "dk", "dv", "dw"), got, want):
         assert torch.isfinite(a).all(), name
         assert (a - b).norm() <= 2.0 ** -7 * b.norm() + 1e-6, name
+
+
+@pytest.mark.parametrize("B,L,Hkv,G,W,inert,odd_rows", [
+    (1, 1, 1, 1, 0, 0, False),           # one row: every streamed row past it repeats it
+    (1, 10, 2, 7, 4, 0, False),          # 70 rows: a second tile of 6
+    (2, 130, 1, 3, 17, 64, False),       # a second key block of 2 keys
+    (1, 257, 3, 2, 300, 64, True),       # every row seen; dK / dV in parts
+    (1, 333, 2, 5, 40, 0, True),         # waves that skip tiles at both window ends
+    (1, 200, 1, 96, 33, 0, False),       # one position spans two tiles
+    (1, 1100, 1, 8, 500, 64, True),      # 8 parts
+    (1, 33000, 1, 1, 33000, 64, False),  # more key tiles than the inert-key table holds
+])
+def test_window_backward_streams_and_parts_vs_float64(B, L, Hkv, G, W, inert, odd_rows):
+    print(f"[gpu-case] window backward B={B} L={L} Hkv={Hkv} G={G} W={W}", flush=True)
+    from mrsa.local_attention import local_attention_autograd, local_attention_backward
+
+    g = torch.Generator().manual_seed(40 + L + G)
+    q, do = (torch.randn(B, L, Hkv * G, 128, generator=g).bfloat16() for _ in range(2))
+    k, v = (torch.randn(B, L, Hkv, 128, generator=g).bfloat16() for _ in range(2))
+    valid = torch.ones(B, L, dtype=torch.bool)
+    if odd_rows:
+        valid = torch.rand(B, L, generator=g) > 0.1
+    if L > 4096:  # (the dense form is too large: one row block's dQ, which reads every key)
+        rows = slice(L - 64, L)
+    else:
+        rows = slice(0, L)
+    ref = [t.to(DEV).double().requires_grad_() for t in (q[:, rows], k, v)]
+    dead = ~valid.to(DEV)
+    i = torch.arange(L, device=DEV)
+    if inert:
+        dead = dead | ((i + 1) % inert == 0)[None]
+    far = (i[rows, None] - i[None]).abs() > W
+    parts, lse = [], []
+    for h in range(Hkv * G):
+        live = (~dead).double()[..., None]
+        s = ref[0][:, :, h] @ (ref[1][:, :, h // G] * live).transpose(1, 2) / 128 ** 0.5
+        s = s.masked_fill(far, float("-inf"))
+        p = torch.softmax(s, -1)
+        lse.append(torch.logsumexp(s.detach(), -1))
+        parts.append(p @ (ref[2][:, :, h // G] * live))
+    out = torch.stack(parts, 2)
+    want = torch.autograd.grad(out, ref, do[:, rows].to(DEV).double())
+    ins = [t.to(DEV).requires_grad_() for t in (q, k, v)]
+    if G <= 8:
+        got, _ = local_attention_autograd(*ins, valid.to(DEV), W, inert)
+        got = torch.autograd.grad(got, ins, do.to(DEV))
+    else:  # (past the forward kernel's heads)
+        got = local_attention_backward(*[t.detach() for t in ins], valid.to(DEV),
+                                       out.detach().bfloat16(), torch.stack(lse, 2).float(),
+                                       do.to(DEV), W, inert)
+    # P and dS are rounded to bf16 before their products and the gradients after
+    # (2^-9 each, independent); D comes from the bf16 output (2^-9 of |dO| |O|)
+    for name, a, b in zip(("dq", "dk", "dv"), got, want):
+        a = a[:, rows].double() if name == "dq" else a.double()
+        assert torch.isfinite(a).all(), name
+        if name == "dq" or L <= 4096:
+            assert (a - b).norm() <= 2.0 ** -7 * b.norm() + 2.0 ** -8 * L ** 0.5, name
