@@ -80,3 +80,36 @@ def test_routed_tiles_and_parts_vs_oracle(B, Lq, C, Hkv, G, K, keep, det):
     # w P rounded to bf16 once per term and the output once: 2^-9 of the row's
     # absolute sum (weights sum to 1, |v| < 5) and of the output
     torch.testing.assert_close(got.cpu().float(), want, atol=5 * 2.0 ** -9, rtol=2.0 ** -8)
+
+
+@pytest.mark.parametrize("C,G,K,keep", [
+    (257, 7, 5, False),      # one chunk past the rule
+    (300, 8, 32, True),
+    (700, 3, 8, False),      # (lists with negative ends and a repeated chunk)
+])
+def test_routed_attention_walks_that_join_vs_oracle(C, G, K, keep):
+    print(f"[gpu-case] joined walks C={C} G={G} K={K} keep={keep}", flush=True)
+    g = torch.Generator().manual_seed(C)
+    Lq, Hkv = 600, 2             # 8-query tiles, whole walks
+    q = torch.randn(1, Lq, Hkv * G, 128, generator=g).bfloat16()
+    k, v = (torch.randn(1, C * 64, Hkv, 128, generator=g).bfloat16() for _ in range(2))
+    w = torch.rand(1, Lq, Hkv * G, K, generator=g).bfloat16()
+    idx = torch.rand(1, Lq, Hkv, C, generator=g).topk(K, -1).indices.sort(-1).values.int()
+    idx[0, 3] = -1               # a query with no chunk
+    idx[0, 5, :, 2:] = -1
+    # descending lists (no chunk twice: the merged slots of a repeated chunk
+    # share the first one's keep row, which the oracle does not)
+    idx[0, 8:16] = idx[0, 8:16].flip(-1)
+    if C == 700:
+        idx[0, 17, :, 1] = idx[0, 17, :, 0]
+    valid = torch.rand(1, C * 64, generator=g) > 0.1
+    tk = (torch.rand(1, Lq, Hkv, K, 64, generator=g) > 0.4).to(torch.int8) if keep else None
+    want = O.selected_attention(q, k, v, w, idx, valid, token_keep=tk).double()
+    frags = kv_fragments(k.to(DEV), v.to(DEV))
+    for _ in range(3):           # each launch joins where the one before it ended
+        got = selected_attention_launch(
+            q.to(DEV), frags, w.to(DEV), idx.to(DEV), valid.to(DEV), 64,
+            token_keep=None if tk is None else tk.to(DEV)).double().cpu()
+        # P w is rounded to bf16 before its product and the output after (2^-9 each)
+        assert (got - want).norm() <= 2.0 ** -8 * want.norm()
+        assert torch.equal(got[0, 3], torch.zeros_like(got[0, 3]))
