@@ -377,14 +377,12 @@ __global__ void __launch_bounds__(kDkvThreads, 2) routed_attn_dkv_kernel(BwdArgs
     for (int i = 0; i < rounds; ++i) {
       const int base = base_of(i);
       const int buf = i & 1;
-      // This wave's rows of the round have landed: the round's entries, loaded
-      // after them, have been read.  The barrier covers the other waves' rows
-      // (and, first, the V and K images), and their reads of the buffers written
-      // next.
+      // This wave's rows of the round have landed; the barrier covers the other
+      // waves' (and, first, the V and K images), and their reads of the buffers
+      // written next.  Wait and barrier are one block: a wait that comes from
+      // the use of a value loaded after the rows may be moved past the barrier.
+      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
       split(evn, entn);
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      __builtin_amdgcn_s_barrier();
-      asm volatile("" ::: "memory");
       uint32_t wraw[2][4];
       load_w(ent, wraw);
       asm volatile("" ::: "memory");
