@@ -440,6 +440,10 @@ __global__ void __launch_bounds__(kDkvThreads, 2) routed_attn_dkv_kernel(BwdArgs
           for (int mt = 0; mt < 2; ++mt)
             x[mt] = alibi(half, mt, r, __builtin_fmaf(S[mt][r], c2, ma[mt]));
           if constexpr (STAB) {
+            // (an excluded key's NaN or infinite logit is not made -inf by the
+            // sum above; without STAB it fails the range test)
+#pragma unroll
+            for (int mt = 0; mt < 2; ++mt) x[mt] = ma[mt] == ninf ? ninf : x[mt];
             const float m = group16_max(fmaxf(x[0], x[1]));
             pmax[r] = m;
             const float mb = m == ninf ? 0.f : m;

@@ -157,3 +157,40 @@ def test_window_backward_streams_and_parts_vs_float64(B, L, Hkv, G, W, inert, od
         assert torch.isfinite(a).all(), name
         if name == "dq" or L <= 4096:
             assert (a - b).norm() <= 2.0 ** -7 * b.norm() + 2.0 ** -8 * L ** 0.5, name
+
+
+@pytest.mark.parametrize("keep,alibi", [(False, False), (True, False), (False, True)])
+@pytest.mark.parametrize("value", [float("nan"), float("inf")])
+def test_routed_backward_ignores_what_excluded_keys_hold(keep, alibi, value):
+    """NaN or infinite K rows of invalid keys reach no gradient but dQ (whose
+    product dS . K meets them with dS = 0)."""
+
+    print(f"[gpu-case] routed backward, {value} in invalid keys keep={keep} alibi={alibi}",
+          flush=True)
+    g = torch.Generator().manual_seed(31)
+    Lq, C, Hkv, G, K = 70, 4, 2, 3, 3
+    r = lambda *s: torch.randn(*s, generator=g).bfloat16()
+    q, do = r(1, Lq, Hkv * G, 128), r(1, Lq, Hkv * G, 128)
+    k, v = r(1, C * 64, Hkv, 128), r(1, C * 64, Hkv, 128)
+    w = torch.rand(1, Lq, Hkv * G, K, generator=g).bfloat16()
+    idx = torch.rand(1, Lq, Hkv, C, generator=g).topk(K, -1).indices.int()
+    valid = torch.rand(1, C * 64, generator=g) > 0.2
+    tk = (torch.rand(1, Lq, Hkv, K, 64, generator=g) > 0.2).to(torch.int8) if keep else None
+    slope = torch.rand(Hkv * G, generator=g) if alibi else None
+
+    def grads(kk):
+        ins = [t.to(DEV).requires_grad_() for t in (q, kk, v, w)]
+        mrsa.HiLS_block_M_head(*ins, idx.to(DEV), key_valid=valid.to(DEV),
+                               token_keep=None if tk is None else tk.to(DEV),
+                               slope=None if slope is None else slope.to(DEV)
+                               ).backward(do.to(DEV))
+        return [t.grad.double().cpu() for t in ins]
+
+    want = grads(k)
+    bad = k.clone()
+    bad[~valid] = value
+    got = grads(bad)
+    # the same terms in another order, each gradient rounded to bf16 once
+    for name, a, b in list(zip(("dq", "dk", "dv", "dw"), got, want))[1:]:
+        assert torch.isfinite(a).all(), name
+        assert (a - b).norm() <= 2.0 ** -8 * b.norm(), name
