@@ -183,10 +183,12 @@ def _split_parts(batch: int, q_len: int, kv_heads: int, kv_len: int, topk: int,
     (4 x 32 queries, 256 chunks: 42 us, 49 with one, 45 with four).
     """
 
-    tile = min(_SEL_TILE_QUERIES, 1024 // topk // 4 * 4)
-    if tile < 4 or q_len == 0 or batch == 0:
-        return 1
     heads = kv_heads * batch
+    if min(topk, chunk_size, heads, q_len) <= 0:  # nothing to split, or refused by the library
+        return 1
+    tile = min(_SEL_TILE_QUERIES, 1024 // topk // 4 * 4)
+    if tile < 4:
+        return 1
     while tile > 4 and -(-q_len // (-(-tile // 8) * 4)) * heads <= 256:
         tile = -(-tile // 8) * 4
     walks = -(-q_len // tile) * heads

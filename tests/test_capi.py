@@ -115,6 +115,27 @@ def test_walk_parts_heuristic():
     assert walk_parts(0, 32, 4, 4096, 32) == 1
 
 
+def test_split_parts_leave_empty_and_refused_sizes_to_the_library():
+    from mrsa.sparse_attention import _split_parts
+
+    for sizes in ((1, 32, 4, 4096, 0, 64), (1, 32, 4, 4096, 32, 0), (1, 16384, 4, 16384, 32, 0),
+                  (0, 32, 4, 4096, 32, 64), (1, 0, 4, 4096, 32, 64), (1, 32, 0, 4096, 32, 64)):
+        assert _split_parts(*sizes) == 1
+
+
+@pytest.mark.gpu
+def test_selected_attention_without_slots_is_a_value_error():
+    import torch
+
+    from mrsa.sparse_attention import selected_attention_launch
+
+    q = torch.zeros(1, 4, 7, 128, dtype=torch.bfloat16, device="cuda:0")
+    frags = torch.zeros(1, 1, 2, 16384, dtype=torch.bfloat16, device="cuda:0")
+    idx = torch.zeros(1, 4, 1, 0, dtype=torch.int32, device="cuda:0")
+    with pytest.raises(ValueError):
+        selected_attention_launch(q, frags, q[..., :0], idx, None, 64)
+
+
 def test_layer_cache_replace_on_host_tensors():
     # fastdllm_cache.py:94-125 on CPU tensors (no tiled copy yet): rows land,
     # errors as in the reference.
