@@ -19,18 +19,25 @@ import torch
 from . import _lib
 from .kernel_utils import group_pad_to
 
-# Largest workspace the route path may take of the 288 GB of HBM (beyond it
-# the scalar general kernel runs).
+# Largest workspace the route path takes by itself of the 288 GB of HBM (beyond
+# it the scalar general kernel runs, unless the caller asks for a workspace).
 _WORKSPACE_LIMIT = 16 << 30
 
 
-def _workspace_bytes(B, L, C, Hkv, G, D, topk, scores_fp32, is_causal):
+def _workspace_bytes(B, L, C, Hkv, G, D, topk, scores_fp32, is_causal, use_workspace=None):
     """Bytes of the workspace the route kernels take, 0 for none: the fp32
     selection scores [B, L, Hkv, C] of many rows against more than 256 chunks
     (1.07 GB for a 64k-token layer with 1024 chunks), the fp32 logits
-    [B, L, Hkv, G, C] of a short block."""
+    [B, L, Hkv, G, C] of a short block.  ``use_workspace`` True takes them at
+    any size; None falls back to the logits where those alone keep the limit
+    (one head per KV head, chunks not a multiple of 16)."""
+    if use_workspace is False:
+        return 0
     n = int(_lib.call("mrsa_route_topk_needed_bytes", B, L, C, Hkv, G, D, topk,
                       1 if is_causal else 0, 1 if scores_fp32 else 0))
+    if use_workspace or n <= _WORKSPACE_LIMIT:
+        return n
+    n = int(_lib.call("mrsa_route_topk_workspace_bytes", B, L, C, Hkv, G))
     return n if n <= _WORKSPACE_LIMIT else 0
 
 
@@ -61,8 +68,8 @@ def route_topk_launch(
     drop mask of remote_drop_mask(key_valid, derive_window, block_size) is
     computed inside the kernel instead.
     Returns indices [B, L, Hkv, topk] int32 and scores [B, L, Hkv, G, topk].
-    ``use_workspace`` (None: by shape) passes the kernels a workspace; the
-    one-pass kernel (up to 256 chunks) takes none.
+    ``use_workspace`` (None: by shape, up to 16 GB) passes the kernels a
+    workspace; the one-pass kernel (up to 256 chunks) takes none.
     """
 
     if selection_mode not in {"post_softmax", "pre_softmax"}:
@@ -193,10 +200,8 @@ def _route_topk_impl(q5, lmks, lse4, bias4, drop_mask, key_valid, topk, block_si
         0 if selection_mode == "post_softmax" else 1, float(sm_scale),
         _lib.ptr(indices), _lib.ptr(scores), 1 if scores_fp32 else 0,
     )
-    nbytes = _workspace_bytes(B, L, C, Hkv, G, D, topk, scores_fp32, is_causal)
-    if use_workspace is None:
-        use_workspace = nbytes > 0
-    if use_workspace:
+    nbytes = _workspace_bytes(B, L, C, Hkv, G, D, topk, scores_fp32, is_causal, use_workspace)
+    if nbytes > 0:
         ws = torch.empty((nbytes + 3) // 4, dtype=torch.float32, device=q5.device)
         st = _lib.call("mrsa_route_topk_ws_fwd", *args, _lib.ptr(ws), nbytes,
                        _lib.stream_of(qc))

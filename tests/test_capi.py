@@ -136,6 +136,48 @@ def test_selected_attention_without_slots_is_a_value_error():
         selected_attention_launch(q, frags, q[..., :0], idx, None, 64)
 
 
+@pytest.mark.parametrize("use_workspace,rows,chunks,groups,limit,entry,nbytes", [
+    # (4 KV heads.)  Up to the limit the path's own bytes: selection scores and
+    # LSE totals of many rows, logits of few, none for up to 256 chunks.
+    (None, 1024, 300, 7, 1 << 34, "ws", 4096 * (304 + 7) * 4),
+    (None, 32, 300, 7, 1 << 34, "ws", 128 * 7 * 300 * 4),
+    (None, 1024, 256, 7, 1 << 34, "plain", 0),
+    (None, 1024, 300, 7, 1 << 20, "plain", 0),
+    # past it only where asked for
+    (True, 1024, 300, 7, 1 << 20, "ws", 4096 * (304 + 7) * 4),
+    (True, 32, 300, 7, 1 << 17, "ws", 128 * 7 * 300 * 4),
+    (False, 32, 300, 7, 1 << 34, "plain", 0),
+    # one head: its logits are the smaller workspace, and alone keep the limit
+    (None, 1024, 300, 1, 4096 * 300 * 4, "ws", 4096 * 300 * 4),
+])
+def test_route_workspace_is_the_callers_choice(monkeypatch, use_workspace, rows, chunks, groups,
+                                               limit, entry, nbytes):
+    import torch
+
+    from mrsa import _lib, topk
+
+    calls = []
+
+    def call(name, *args):
+        if name.endswith("_bytes"):
+            return real(name, *args)
+        calls.append((name, args))
+        return 0
+
+    real = _lib.call
+    monkeypatch.setattr(_lib, "call", call)
+    monkeypatch.setattr(_lib, "stream_of", lambda t: None)
+    monkeypatch.setattr(topk, "_WORKSPACE_LIMIT", limit)
+    q = torch.zeros(1, rows, 4, groups, 128, dtype=torch.bfloat16)
+    lmk = torch.zeros(1, chunks, 4, 128, dtype=torch.bfloat16)
+    topk._route_topk_impl(q, lmk, None, None, None, None, 32, 64, -1, False, 0, 0, True, 1.0,
+                          False, -1 if use_workspace is None else int(use_workspace))
+    (name, args), = calls
+    assert name == {"ws": "mrsa_route_topk_ws_fwd", "plain": "mrsa_route_topk_fwd"}[entry]
+    if entry == "ws":
+        assert args[-2] == nbytes and args[-3]
+
+
 def test_layer_cache_replace_on_host_tensors():
     # fastdllm_cache.py:94-125 on CPU tensors (no tiled copy yet): rows land,
     # errors as in the reference.
