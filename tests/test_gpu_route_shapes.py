@@ -113,3 +113,48 @@ def test_routed_attention_walks_that_join_vs_oracle(C, G, K, keep):
         # P w is rounded to bf16 before its product and the output after (2^-9 each)
         assert (got - want).norm() <= 2.0 ** -8 * want.norm()
         assert torch.equal(got[0, 3], torch.zeros_like(got[0, 3]))
+
+
+@pytest.mark.parametrize("mu", [2.0, 6.0, 12.0])
+def test_route_scores_order_near_ties_as_well_as_the_plain_fp32_form(mu):
+    """Two chunks whose scores, each another head's, lie within 1e-6: picks that
+    differ from 64 bits are no more than those of x - logaddexp(LSE, m + log(sum
+    of exp(x - m))) with each step rounded to fp32."""
+
+    print(f"[gpu-case] route near ties mu={mu}", flush=True)
+    L, H = 16384, 4
+    g = torch.Generator().manual_seed(int(mu))
+    a = (0.5 + 3.5 * torch.rand(L, H, 2, generator=g)).bfloat16()
+    # head i's logits: a_i at chunk i, -8 a_i at the other (exact products)
+    x = torch.stack([torch.stack([a[..., 0], -8 * a[..., 0]], -1),
+                     torch.stack([-8 * a[..., 1], a[..., 1]], -1)], -2).float()
+    l64 = torch.logsumexp(x.double(), -1)
+    lse = torch.empty(L, H, 2)
+    lse[..., 0] = mu + 0.5 * torch.randn(L, H, generator=g)
+    total0 = torch.logaddexp(lse[..., 0].double(), l64[..., 0])
+    total1 = a[..., 1].double() - (a[..., 0].double() - total0) \
+        + 2e-6 * (torch.rand(L, H, generator=g, dtype=torch.float64) - 0.5)
+    lse[..., 1] = total1 + torch.log(-torch.expm1(l64[..., 1] - total1))
+    assert torch.isfinite(lse).all()
+
+    def picks(total):  # of the larger of the heads' maxima, ties to chunk 0
+        s = (x.to(total.dtype) - total[..., None]).amax(-2)
+        return (s[..., 1] > s[..., 0]).int()
+
+    exact = picks(torch.logaddexp(lse.double(), l64))
+    m = x.amax(-1)
+    plain = m + torch.log(torch.exp(x - m[..., None]).sum(-1))
+    hi, lo = torch.maximum(lse, plain), torch.minimum(lse, plain)
+    worst = int((picks(hi + torch.log1p(torch.exp(lo - hi))) != exact).sum())
+
+    q = torch.zeros(1, L, H, 2, 128, dtype=torch.bfloat16)
+    q[0, ..., 0] = a
+    lmk = torch.zeros(1, 2, H * 2, 128, dtype=torch.bfloat16)
+    lmk[0, 0, :, 0] = torch.tensor([1.0, -8.0]).repeat(H)
+    lmk[0, 1, :, 0] = torch.tensor([-8.0, 1.0]).repeat(H)
+    idx, _ = route_topk_launch(q.to(DEV), lmk.to(DEV), lse[None].to(DEV), 1, 64, sm_scale=1.0)
+    got = int((idx[0, ..., 0].cpu() != exact).sum())
+    print(f"picks off 64 bits: {got}, plain form {worst} of {L * H}")
+    # 4000 to 14000 of 65536 differ: 10% is six standard deviations or more (the
+    # totals held in base 2 give 20% to 40% more)
+    assert got <= 1.1 * worst
