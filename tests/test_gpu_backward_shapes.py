@@ -159,6 +159,41 @@ def test_window_backward_streams_and_parts_vs_float64(B, L, Hkv, G, W, inert, od
             assert (a - b).norm() <= 2.0 ** -7 * b.norm() + 2.0 ** -8 * L ** 0.5, name
 
 
+@pytest.mark.parametrize("C,alibi", [(257, False), (300, True)])
+def test_routed_backward_walks_that_join_vs_oracle(C, alibi):
+    """Past 256 chunks the dQ walk (and the ALiBi forward) start where other
+    walks are."""
+
+    print(f"[gpu-case] routed backward, joined walks C={C} alibi={alibi}", flush=True)
+    g = torch.Generator().manual_seed(C)
+    Lq, Hkv, G, K = 300, 2, 3, 6
+    r = lambda *s: torch.randn(*s, generator=g).bfloat16()
+    q, do = r(1, Lq, Hkv * G, 128), r(1, Lq, Hkv * G, 128)
+    k, v = r(1, C * 64, Hkv, 128), r(1, C * 64, Hkv, 128)
+    w = torch.rand(1, Lq, Hkv * G, K, generator=g).bfloat16()
+    idx = torch.rand(1, Lq, Hkv, C, generator=g).topk(K, -1).indices.int()  # any order
+    idx[0, 3] = -1
+    idx[0, 5, :, 2:] = -1
+    idx[0, 10:40, :, 4] = idx[0, 10:40, :, 1]   # a chunk twice
+    valid = torch.rand(1, C * 64, generator=g) > 0.1
+    slope = torch.rand(Hkv * G, generator=g) if alibi else None
+
+    ref = [t.float().requires_grad_() for t in (q, k, v, w)]
+    out = O.selected_attention(*ref, idx, valid, slope=slope)
+    want = [out.detach()] + list(torch.autograd.grad(out, ref, do.float()))
+    for _ in range(3):           # each launch joins where the one before it ended
+        ins = [t.to(DEV).requires_grad_() for t in (q, k, v, w)]
+        out = mrsa.HiLS_block_M_head(*ins, idx.to(DEV), key_valid=valid.to(DEV),
+                                     slope=None if slope is None else slope.to(DEV))
+        got = [out.detach()] + list(torch.autograd.grad(out, ins, do.to(DEV)))
+        # the bounds of test_routed_backward_splits_vs_oracle; a repeated chunk's
+        # weights are added in bf16 first (2^-9 more)
+        for name, a, b in zip(("out", "dq", "dk", "dv", "dw"), got, want):
+            a, b = a.double().cpu(), b.double()
+            assert torch.isfinite(a).all(), name
+            assert (a - b).norm() <= 2.0 ** -7 * b.norm(), name
+
+
 @pytest.mark.parametrize("keep,alibi", [(False, False), (True, False), (False, True)])
 @pytest.mark.parametrize("value", [float("nan"), float("inf")])
 def test_routed_backward_ignores_what_excluded_keys_hold(keep, alibi, value):

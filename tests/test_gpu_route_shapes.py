@@ -10,6 +10,7 @@ from oracle import mrsa_oracle as O
 pytestmark = pytest.mark.gpu
 
 if torch.cuda.is_available():
+    import mrsa
     from mrsa.sparse_attention import kv_fragments, selected_attention_launch
     from mrsa.topk import route_topk_launch
 
@@ -29,6 +30,8 @@ NEAR_TIE = 1e-5
     (1, 1025, 257, 4, 7, 32),      # scan path: C = 1 mod 16 and 64
     (2, 683, 304, 3, 3, 24),
     (1, 4099, 320, 1, 8, 64),
+    (1, 4097, 2049, 1, 2, 24),     # one chunk past the pick's 32-per-lane instance
+    (2, 2050, 4096, 1, 1, 64),     # the most chunks
 ])
 def test_route_topk_tile_edges_vs_oracle(B, L, C, Hkv, G, topk):
     print(f"[gpu-case] route tile edges B={B} L={L} C={C} Hkv={Hkv} G={G} K={topk}", flush=True)
@@ -51,6 +54,42 @@ def test_route_topk_tile_edges_vs_oracle(B, L, C, Hkv, G, topk):
     # the sums' own difference (below 1e-3 at these magnitudes)
     torch.testing.assert_close(sc.cpu().float()[ok], rsc.bfloat16().float()[ok], atol=2e-3,
                                rtol=2.0 ** -8)
+
+
+@pytest.mark.parametrize("C,Hkv,G,topk,window,valid_keys", [
+    (257, 1, 7, 32, 100, True),    # one chunk past the one-pass kernels
+    (271, 2, 2, 8, 319, True),     # neither a multiple of 16 nor of 64
+    (304, 1, 3, 64, 0, False),     # each query's own chunk alone
+    (290, 1, 1, 20, 30000, True),  # a window that hides every chunk
+])
+def test_route_topk_scan_derived_drop_equals_explicit(C, Hkv, G, topk, window, valid_keys):
+    """The scan path's own drop mask (chunks in the window, chunks with no valid
+    key) against the explicit one and the oracle."""
+
+    print(f"[gpu-case] scan derived drop C={C} Hkv={Hkv} G={G} K={topk} W={window}", flush=True)
+    g = torch.Generator().manual_seed(3000 + C)
+    B, L = 2, 64 * C
+    q5 = torch.randn(B, L, Hkv, G, 128, generator=g).bfloat16()
+    lmk = (0.5 * torch.randn(B, C, Hkv * G, 128, generator=g)).bfloat16()
+    lse4 = torch.randn(B, L, Hkv, G, generator=g) + 3.0
+    bias4 = torch.randn(B, C, Hkv, G, generator=g)
+    valid = torch.ones(B, L, dtype=torch.bool)
+    if valid_keys:
+        valid = torch.rand(B, L, generator=g) > 0.1
+        dead = torch.rand(B, C, generator=g) < 0.2     # chunks with no key, the last one too
+        dead[0, -1] = True
+        dead = dead.repeat_interleave(64, 1)
+        dead[:, 63::64] = False                        # (their landmark slots do not count)
+        valid &= ~dead
+    drop = O.remote_drop_mask(valid, window, 64)
+    args = (q5.to(DEV), lmk.to(DEV), lse4.to(DEV), topk, 64)
+    idx, sc = route_topk_launch(*args, bias4=bias4.to(DEV), derive_window=window,
+                                key_valid=valid.to(DEV) if valid_keys else None)
+    eidx, esc = route_topk_launch(*args, bias4=bias4.to(DEV), drop_mask=drop.to(DEV))
+    assert torch.equal(idx, eidx) and torch.equal(sc, esc)
+    ridx, rsc, sel = O.route_topk(q5, lmk, lse4, topk, 64, drop_mask=drop, bias4=bias4)
+    bad = (idx.cpu().long() != ridx).any(-1)
+    assert int((bad & ~(O.boundary_gap(sel, topk) < NEAR_TIE)).sum()) == 0
 
 
 @pytest.mark.parametrize("B,Lq,C,Hkv,G,K,keep,det", [
@@ -158,3 +197,24 @@ def test_route_scores_order_near_ties_as_well_as_the_plain_fp32_form(mu):
     # 4000 to 14000 of 65536 differ: 10% is six standard deviations or more (the
     # totals held in base 2 give 20% to 40% more)
     assert got <= 1.1 * worst
+
+
+def test_candidate_token_scores_walks_that_join_vs_oracle():
+    print("[gpu-case] joined walks, token scores", flush=True)
+    g = torch.Generator().manual_seed(261)
+    Lq, C, Hkv, G, K = 200, 261, 2, 7, 8
+    q = torch.randn(1, Lq, Hkv * G, 128, generator=g).bfloat16()
+    k = torch.randn(1, C * 64, Hkv, 128, generator=g).bfloat16()
+    idx = torch.rand(1, Lq, Hkv, C, generator=g).topk(K, -1).indices.sort(-1).values.int()
+    idx[0, 3] = -1
+    idx[0, 5, :, 2:] = -1
+    valid = torch.rand(1, C * 64, generator=g) > 0.1
+    want = O.candidate_token_scores(q, k, idx, valid, 64)
+    fin = torch.isfinite(want)
+    for _ in range(3):           # each launch joins where the one before it ended
+        got = mrsa.candidate_token_scores_gqa(q.to(DEV), k.to(DEV), idx.to(DEV), valid.to(DEV),
+                                              64).cpu()
+        assert torch.equal(fin, torch.isfinite(got))
+        # fp32 sums of 128 exact products: 128 x 2^-24 of their absolute sum, near
+        # 128 x 0.64 / sqrt(128)
+        torch.testing.assert_close(got[fin], want[fin], atol=1e-4, rtol=0)
