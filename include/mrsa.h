@@ -267,10 +267,10 @@ int mrsa_route_topk_ws_fwd(const void* q, const void* lmk, const float* lse_loca
  * tight serving loops, harnesses that forbid hipMalloc), e.g. the cached
  * block step's routing over up to 4096 landmarks.
  *   Arguments as mrsa_route_topk_ws_fwd minus the workspace; same results.
- *   Returns MRSA_ERR_SCRATCH when the short-block path (more than 256
- *   chunks) needs more than MRSA_ROUTE_TOPK_SCRATCH_BYTES of fp32 logits
- *   (batch * seq_len * kv_heads * groups * chunks * 4 bytes); shapes of the
- *   matrix-core path (up to 256 chunks) need none.
+ *   Returns MRSA_ERR_SCRATCH when the fp32 logits (batch * seq_len * kv_heads
+ *   * groups * chunks * 4 bytes) pass MRSA_ROUTE_TOPK_SCRATCH_BYTES, whether or
+ *   not the path taken would write them; 7 or 8 groups with the one-pass
+ *   kernel's other limits (up to 256 chunks) are never refused.
  *   Every call on a GPU shares that GPU's buffer: calls that overlap on one
  *   GPU (other streams, other threads) race.
  */

@@ -2351,14 +2351,13 @@ extern "C" int mrsa_route_topk_noalloc_fwd(
     int scores_fp32, void* stream) {
   if (batch < 0 || seq_len < 0 || chunks <= 0 || kv_heads <= 0 || groups <= 0)
     return MRSA_ERR_INVALID_ARGUMENT;
-  // Workspace the workspace entry point takes for this problem: the fp32
-  // logits [batch, seq_len, kv_heads, groups, chunks] of the short-block path.
-  // The one-pass matrix-core path runs without one (the dispatcher's own
-  // test decides).  A problem that needs more than the static buffer is
-  // rejected (by this rule also where the call would take less of it).
-  const int64_t need = groups >= 7 && fast_path(q, lmk, chunks, kv_heads, groups, head_dim, topk, is_causal, scores_fp32)
-                           ? 0
-                           : batch * seq_len * kv_heads * groups * chunks * 4;
+  // What the caller may rely on is the size of the fp32 logits [batch, seq_len,
+  // kv_heads, groups, chunks], except for the one-pass kernel with 7 or 8
+  // groups: larger problems are refused also where the call would take less
+  // (the one-pass kernel with fewer groups, the scan path).
+  const bool one_pass = groups >= 7 && fast_path(q, lmk, chunks, kv_heads, groups, head_dim, topk,
+                                                 is_causal, scores_fp32);
+  const int64_t need = one_pass ? 0 : batch * seq_len * kv_heads * groups * chunks * 4;
   if (need > (int64_t)MRSA_ROUTE_TOPK_SCRATCH_BYTES) return MRSA_ERR_SCRATCH;
   void* ws = nullptr;
   if (need > 0) {

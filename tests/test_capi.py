@@ -115,6 +115,44 @@ def test_walk_parts_heuristic():
     assert walk_parts(0, 32, 4, 4096, 32) == 1
 
 
+@pytest.mark.parametrize("batch,q_len,kv_heads,chunks,topk,parts", [
+    (1, 16384, 4, 256, 32, 1),     # whole walks fill the chip
+    (1, 32, 4, 128, 32, 8),        # a cached block step
+    (1, 32, 4, 2048, 32, 4),       # against a long cache
+    (4, 32, 4, 256, 32, 2),
+    (1, 3, 4, 2048, 4, 3),         # 12 steps: parts of 4
+    (1, 1, 1, 1, 1, 1),
+    (1, 640, 4, 10, 32, 1),
+    (1, 32, 4, 64, 257, 1),        # tiles of fewer than 4 queries are not the kernel's
+    (2, 100, 8, 300, 256, None),
+    (1, 77, 1, 8192, 64, None),
+    (1, 255, 3, 33, 20, None),
+])
+def test_split_parts_agree_with_the_kernels_tiles(batch, q_len, kv_heads, chunks, topk, parts):
+    from mrsa.sparse_attention import _split_parts
+
+    got = _split_parts(batch, q_len, kv_heads, 64 * chunks, topk, 64)
+    assert parts is None or got == parts
+    assert 1 <= got <= 64
+    if got == 1:
+        return
+
+    def kernel_tile(parts):  # the launcher's rule (routed_attention.hip)
+        tile = min(32, 1024 // topk // 4 * 4)
+        while True:
+            half = (tile // 2 + 3) // 4 * 4
+            if half >= tile or batch * kv_heads * parts * -(-q_len // half) > 256:
+                return tile
+            tile = half
+
+    # the parts were chosen for the tile the kernel then takes, one workgroup
+    # per CU, with 4 steps or more
+    assert kernel_tile(got) == kernel_tile(1)
+    tile = kernel_tile(got)
+    assert batch * kv_heads * got * -(-q_len // tile) <= 256
+    assert got <= min(chunks, min(tile, q_len) * topk) // 4
+
+
 def test_split_parts_leave_empty_and_refused_sizes_to_the_library():
     from mrsa.sparse_attention import _split_parts
 

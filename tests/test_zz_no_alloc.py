@@ -106,3 +106,22 @@ def test_no_alloc_route_topk_off_the_matrix_core_path(case):
         assert torch.equal(sc.view(torch.int16), rsc.view(torch.int16))
         rows = rows // 2  # the second call smaller
         q, lse, drop = q[:, :rows], lse[:, :rows].contiguous(), drop[:, :rows].contiguous()
+
+
+def test_no_alloc_route_topk_size_rule_with_few_heads():
+    # Fewer than 7 heads per KV head are held to the logits' size also where the
+    # one-pass kernel, which writes none, takes the call.
+    for rows, refused in ((1024, False), (8200, True)):
+        inp = _inputs(rows, 128, 21, G=4)
+        print(f"[gpu-case] no-alloc route topk, 4 heads: rows={rows}", flush=True)
+        assert (rows * 4 * 4 * 128 * 4 > SCRATCH_BYTES) == refused
+        st, idx, sc = _call("mrsa_route_topk_noalloc_fwd", *inp)
+        if refused:
+            assert st == _lib.MRSA_ERR_SCRATCH
+            continue
+        assert st == 0, _lib.status_string(st)
+        st, ridx, rsc = _call("mrsa_route_topk_ws_fwd", *inp, ws=_workspace(rows, 128, G=4))
+        assert st == 0, _lib.status_string(st)
+        torch.cuda.synchronize()
+        assert torch.equal(idx, ridx)
+        assert torch.equal(sc.view(torch.int16), rsc.view(torch.int16))
