@@ -1,6 +1,6 @@
-// Shared pieces of the window-attention kernel: asm LDS operand reads with
-// explicit waits, and the S^T = K.Q^T product of one 16-column tile over a
-// 64-key tile held in an LDS slot.
+// Shared pieces of the window-attention and backward kernels: asm LDS operand
+// reads with explicit waits, the S^T = K.Q^T product of one 16-column tile over
+// a 64-key tile held in an LDS slot, and transposing LDS reads.
 //
 // Slot layout (32 KB): the tile's K / V fragments (mrsa_kv_fragments): 32
 // operand images of 1 KB, lane l's 16 bytes at 16 l; K image 4 mt + ks holds
@@ -34,6 +34,21 @@ __device__ __forceinline__ void lds_wait(u32x4_t& v) {
 }
 __device__ __forceinline__ uint32_t lds_addr(const void* p) {
   return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p;
+}
+
+typedef short s16x4_t __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) s16x4_t lds_s16x4_t;
+
+// Four 16-bit values of one column out of four LDS rows (gfx950's transposing
+// read): lanes 16 g + i of a group point at 8-byte pieces, piece i & 3 of row
+// i >> 2; lane i receives element i of the four rows.
+__device__ __forceinline__ u32x2_t read_transposed(uint32_t addr) {
+  return __builtin_bit_cast(u32x2_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                                         (lds_s16x4_t*)(uintptr_t)addr));
+}
+// 16 bytes at an LDS address, scheduled and waited for by the compiler.
+__device__ __forceinline__ u32x4_t lds_read16(uint32_t addr) {
+  return *(const __attribute__((address_space(3))) u32x4_t*)(uintptr_t)addr;
 }
 
 template <int N, class F, int... I>

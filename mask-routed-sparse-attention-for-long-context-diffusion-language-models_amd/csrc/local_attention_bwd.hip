@@ -48,20 +48,6 @@ constexpr int kSlotBytes = 2 * kTileBytes;
 constexpr int kMaskTiles = 512;       // inert-key words of the dQ pass kept in LDS
 constexpr int kMaxParts = 8;          // row parts of the dK/dV pass
 
-typedef short s16x4_t __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) s16x4_t lds_s16x4_t;
-
-// Four 16-bit values of one column out of four LDS rows: lanes 16 g + i of a
-// group point at 8-byte pieces, piece i & 3 of row i >> 2; lane i receives
-// element i of the four rows.
-__device__ __forceinline__ u32x2_t read_transposed(uint32_t addr) {
-  return __builtin_bit_cast(u32x2_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                                         (lds_s16x4_t*)(uintptr_t)addr));
-}
-__device__ __forceinline__ u32x4_t lds_read16(uint32_t addr) {
-  return *(const __attribute__((address_space(3))) u32x4_t*)(uintptr_t)addr;
-}
-
 // Buffer resource of `bytes` bytes at a wave-uniform address, in scalar registers.
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t row_rsrc(const uint16_t* at, int bytes) {
   return __builtin_amdgcn_make_buffer_rsrc((void*)uniform_u64((uint64_t)at), (short)0,
@@ -123,7 +109,7 @@ template <bool DKV>
 __global__ void __launch_bounds__(kThreads, DKV ? 2 : 4) local_bwd_kernel(BwdArgs a) {
   extern __shared__ __align__(256) unsigned char smem[];
   unsigned char* ring = smem;
-  uint64_t* inert_tab = reinterpret_cast<uint64_t*>(smem + kRing * kSlotBytes);  // [kMaskTiles]
+  uint64_t* inert_tab = reinterpret_cast<uint64_t*>(smem + kRing * kSlotBytes);  // [kMaskTiles], dQ pass
 
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -150,7 +136,6 @@ __global__ void __launch_bounds__(kThreads, DKV ? 2 : 4) local_bwd_kernel(BwdArg
   bool cok;
   int64_t rlo, rhi;           // visible rows [rlo, rhi] (tile-row units)
   float lse2_c = 0.f, d_c = 0.f;
-  int64_t nrows;              // rows of the streamed sequence
   int64_t cq = 0, cj = 0;
   int cg = 0;
   if constexpr (!DKV) {
@@ -158,7 +143,6 @@ __global__ void __launch_bounds__(kThreads, DKV ? 2 : 4) local_bwd_kernel(BwdArg
     cq = blk * QB + cw / G;
     cg = cw % G;
     cok = cw < QB * G && cq < L;
-    nrows = L;
     rlo = max(cq - W, (int64_t)0);
     rhi = min(cq + W, L - 1);
     const int64_t row = ((b * L + cq) * Hq + (int64_t)h * G + cg) * 128;
@@ -189,7 +173,6 @@ __global__ void __launch_bounds__(kThreads, DKV ? 2 : 4) local_bwd_kernel(BwdArg
   } else {
     cj = blk * 128 + cw;
     cok = cj < L;
-    nrows = L * G;
     rlo = G * max(cj - W, (int64_t)0);
     rhi = G * min(cj + W, L - 1) + G - 1;
     const int64_t row = ((b * L + (cok ? cj : 0)) * a.Hkv + h) * 128;
@@ -592,7 +575,7 @@ extern "C" int mrsa_local_attention_bwd(const void* q, const void* k, const void
   a.dq = grad_q;
   a.dk = grad_k;
   a.dv = grad_v;
-  const size_t smem = (size_t)kRing * kSlotBytes + kMaskTiles * 8;
+  const size_t ring = (size_t)kRing * kSlotBytes, smem = ring + kMaskTiles * 8;
   if (hipFuncSetAttribute(reinterpret_cast<const void*>(local_bwd_kernel<false>),
                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess)
     return MRSA_ERR_LAUNCH;
@@ -603,12 +586,12 @@ extern "C" int mrsa_local_attention_bwd(const void* q, const void* k, const void
   int st = mrsa_launch_status();
   if (st != MRSA_OK) return st;
   if (hipFuncSetAttribute(reinterpret_cast<const void*>(local_bwd_kernel<true>),
-                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess)
+                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)ring) != hipSuccess)
     return MRSA_ERR_LAUNCH;
   hipLaunchKernelGGL(local_bwd_kernel<true>,
                      dim3((unsigned)((seq_len + 127) / 128 * a.parts), (unsigned)kv_heads,
                           (unsigned)batch),
-                     dim3(kThreads), smem, s, a);
+                     dim3(kThreads), ring, s, a);
   st = mrsa_launch_status();
   if (st != MRSA_OK || a.parts == 1) return st;
   const int64_t n4 = batch * seq_len * kv_heads * 32;

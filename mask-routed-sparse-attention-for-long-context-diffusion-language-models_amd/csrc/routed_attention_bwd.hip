@@ -33,6 +33,7 @@
 //   fwd = mrsa_kv_fragments(k, v): K images (keys x dims) for S^T = K . Q^T;
 //   bwd = mrsa_kv_fragments(v, k): V images (keys x dims) for dP^T = V . dO^T
 //         and K^T images (dims x keys, tiled order) for the walk's dS . K.
+#include "chunk_tile.h"
 #include "mrsa_device.h"
 
 #include <algorithm>
@@ -188,25 +189,6 @@ __global__ void __launch_bounds__(kListBlock) list_fill_kernel(BwdArgs a, const 
       list[(int64_t)a.start[bhc] + blkbase[(bh * nqb + qb) * a.Ck + c] + p] =
           (int32_t)(q | ((int64_t)k << 24));
     });
-}
-
-typedef __attribute__((address_space(3))) void lds_void_t;
-typedef short s16x4_t __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) s16x4_t lds_s16x4_t;
-
-// Four 16-bit values of one column out of four LDS rows (gfx950's transposing
-// read): lanes 16 g + i of a group point at 8-byte pieces, piece i & 3 of row
-// i >> 2; lane i receives element i of the four rows.
-__device__ __forceinline__ u32x2_t read_transposed(uint32_t addr) {
-  return __builtin_bit_cast(u32x2_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                                         (lds_s16x4_t*)(uintptr_t)addr));
-}
-__device__ __forceinline__ uint32_t lds_addr(const void* p) {
-  return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) char*)(p);
-}
-
-__device__ __forceinline__ u32x4_t lds_read16(uint32_t addr) {
-  return *(const __attribute__((address_space(3))) u32x4_t*)(uintptr_t)addr;
 }
 
 // One workgroup per work unit: chunk (b, h, c) and a segment of its pairs.  8
