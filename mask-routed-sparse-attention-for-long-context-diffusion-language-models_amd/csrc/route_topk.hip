@@ -320,10 +320,12 @@ __global__ void __launch_bounds__(kHeadThreads, 4)
     }
     // LSE over all chunks with the hardware exp2 / log2.  With every x -inf the
     // stabiliser is 0 and the sum 0.  The terms are 2^(x log2e - m2) with m2 =
-    // m log2e rounded; the rounding goes back in as fma(-m, log2e, m2), so that
-    // the LSE is as close as m + logf(sum of expf(x - m)) is (scores' rms error
-    // over 3..256 chunks 0.9..1.02 times that form's; 1..1.5 with the LSE held
-    // in base 2).
+    // m log2e rounded.  With up to 6 heads the rounding goes back in as
+    // fma(-m, log2e, m2), so that the LSE is as close as the short-block path's
+    // m + logf(sum of expf(x - m)) (scores' rms error over 3..256 chunks 0.9..1.02
+    // times that form's; 1..1.5 with the LSE held in base 2).  With 7 or 8 it
+    // stays in base 2 as route_tile_kernel holds it: which of the two kernels
+    // takes a call depends on its length, and near ties fall the same way.
 #pragma unroll
     for (int u = 0; u < QT; ++u) tot[u] = 0.f;
     if (!a.pre_softmax) {  // uniform
@@ -362,9 +364,12 @@ __global__ void __launch_bounds__(kHeadThreads, 4)
         part[u] = across4_sum((p[u][0] + p[u][1]) + (p[u][2] + p[u][3]));
 #pragma unroll
       for (int u = 0; u < QT; ++u)
-        tot[u] = route_total_ln(
-            lse[u], __builtin_fmaf(log2_hw(part[u]) + __builtin_fmaf(-m[u], kLog2e, m2[u]), kLn2,
-                                   m[u]));
+        if (G >= 7) {  // uniform
+          tot[u] = route_total(lse[u], m2[u] + log2_hw(part[u]));
+        } else {
+          const float back = __builtin_fmaf(-m[u], kLog2e, m2[u]);
+          tot[u] = route_total_ln(lse[u], __builtin_fmaf(log2_hw(part[u]) + back, kLn2, m[u]));
+        }
     }
   }
   __syncthreads();  // the rings are done
