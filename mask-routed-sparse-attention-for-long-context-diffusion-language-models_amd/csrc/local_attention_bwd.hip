@@ -25,12 +25,14 @@
 // The dQ pass also writes each (query, head) row's lse (log2 units) and D in
 // row order for the dK/dV pass.
 //
-// Bound: LDS operand reads (64 KB a tile and wave in the dK/dV pass, 4096 of
-// its cycles at 128 B / clock, twice the products').  Operands read 4 (dQ) or 8
-// ahead by explicit order; the dQ pass fits 128 registers and 64 KB of LDS, so
-// that two workgroups share a CU.  28 heads over 4, 16384 queries, window 319:
-// dQ 365 us, dK/dV 443; with pre-transposed images in HBM (four layout
-// launches, 214 us) and 64 KB slots, one workgroup per CU, 473 and 527.
+// No unit is at its limit (dQ / dK/dV pass, 28 heads over 4, 5003 queries, window
+// 1280): LDS is busy 67 / 47% of the cycles, 40 / 33% of that bank conflicts, the
+// matrix cores work 40 / 31%, and the waves wait 34 / 35% of their time, at the
+// tile's barrier and for its rows and operands.  Operands read 4 (dQ) or 8
+// ahead by explicit order; the dQ pass fits 128 registers and 68 KB of LDS, so
+// that two workgroups share a CU.  16384 queries, window 319: dQ 330-365 us,
+// dK/dV 407-443; with pre-transposed images in HBM (four layout launches, 214
+// us) and 64 KB slots, one workgroup per CU, 473 and 527.
 #include "chunk_tile.h"
 #include "mrsa_device.h"
 
@@ -492,10 +494,9 @@ BwdPlan bwd_plan(int64_t B, int64_t L, int64_t Hkv, int64_t G) {
 // Row parts of the dK/dV pass.  A workgroup (128 keys) has a CU to itself, so
 // the launch takes ceil(units parts / 256) rounds of its tiles / parts, each
 // with about 6 tiles' time around the loop; a part writes and reads back 2 KB
-// per key row, a tile's time (2.5 us) for 10 MB.
-// 5003 keys, window 1280 (160 workgroups of 295 tiles): 543 us in 3 parts with
-// 13 for their sum, 780 whole (in the pre-transposed form; 1.2 times less in
-// this one at whole rounds).
+// per key row, a tile's time (2.3 us) for 10 MB.
+// 5003 keys, window 1280 (160 workgroups of 295 tiles): 470 us in 3 parts and 14
+// for their sum, 664 whole; 2 x 1984 keys, window 319: 103 + 8 us, 184 whole.
 int pick_parts(const BwdPlan& p, int64_t B, int64_t L, int64_t Hkv, int64_t G, int64_t W) {
   const int64_t units = key_blocks(B, L, Hkv);
   const int64_t tiles = (G * std::min(L, 128 + 2 * std::min(W, L)) + 63) / 64;

@@ -992,11 +992,12 @@ __global__ void __launch_bounds__(kTileThreads, 1) route_tile_kernel(RouteArgs a
 // the 64 -- here 4 pairs per lane and query, so that near ties between heads
 // fall the same way as they always did.
 //
-// Measured at 65536 queries x 4 KV heads x 7 heads against 1024 chunks: 1640
-// (LSE) + 1170 (scan) + 1440 (pick) us; 7590 + 6260 us with the fp32 logits of
-// every head through memory (7.5 GB written and read).  The LSE kernel is bound
-// by the ~25 VALU instructions of each term, the scan by its products and
-// their 7-head epilogue at two waves per SIMD, the pick by the gather.
+// Measured at 65536 queries x 4 KV heads x 7 heads against 1024 chunks: 1490-1640
+// (LSE) + 1140-1170 (scan) + 1350-1440 (pick) us; 7590 + 6260 us with the fp32
+// logits of every head through memory (7.5 GB written and read).  The LSE kernel
+// is bound by the ~30 VALU instructions of each term (the VALU never idles); the
+// scan (VALU 43%, matrix cores 18%, waves waiting 35%) by its products and their
+// 7-head epilogue at two waves per SIMD; the pick (waiting 50%) by the gather.
 // ---------------------------------------------------------------------------
 constexpr int kScanThreads = 512;
 constexpr int kScanQ = 128;

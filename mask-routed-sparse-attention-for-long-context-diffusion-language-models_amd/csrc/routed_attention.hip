@@ -84,8 +84,10 @@ __device__ unsigned long long g_lock_giveups;
 
 // Per XCD (128 bytes apart): the furthest chunk its workgroups have walked to,
 // counted on over the laps.  Only a hint where a new walk joins the running
-// ones, read and raised without order by every launch; any value gives the
-// same terms.
+// ones, read and raised without order by every launch on any stream; any value
+// gives the same terms.  The order of a row's fp32 additions past kJoinChunks
+// thus depends on earlier launches too; it was never fixed there (waves add as
+// they take the row lock), and the fixed-order mode does not join.
 __device__ unsigned long long g_walk_at[8 * 16];
 
 namespace {

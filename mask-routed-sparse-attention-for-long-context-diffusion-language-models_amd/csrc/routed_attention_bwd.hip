@@ -205,12 +205,14 @@ __global__ void __launch_bounds__(kListBlock) list_fill_kernel(BwdArgs a, const 
 // the rest and V in LDS, its dK and dV (32 keys x 128 dims, fp32) in 128 accumulators, summed
 // over the four groups through LDS once per unit.  Halving the keys and not
 // the pairs is what lets two waves share a SIMD; with 64 keys per wave the 256
-// accumulators left no registers and the kernel ran 5090 us.  Bound: the Q and
-// dO rows, read once per routed slot (7.5 GB at 16384 queries x 28 heads x 32
-// slots, 60% of it past L2) beside 1.9 GB of records written; products and
-// VALU instructions take 55% of the cycles, LDS 26%.  Measured there: 2270 us;
-// with eight pairs per workgroup and round, element-wise transposes through LDS
-// and no prefetch 3410 us.
+// accumulators left no registers and the kernel ran 5090 us.  No unit is at its
+// limit at 16384 queries x 28 heads x 32 slots: the matrix cores work 21% of the
+// cycles, the VALU 43% (products included), LDS 31%; 8.4 GB read (the Q and dO
+// rows, once per routed slot) and 2.7 GB written make 4.9 TB/s.  The waves wait
+// 39% of their time, at a round's two barriers and for the rows, and two of them
+// per SIMD do not cover it.  Measured there: 2270 us; with eight pairs per
+// workgroup and round, element-wise transposes through LDS and no prefetch
+// 3410 us.
 constexpr int kGroups = 4;                 // pair groups of a workgroup
 constexpr int kDkvThreads = 128 * kGroups;
 constexpr int kPairs = 4;                  // per group and round
